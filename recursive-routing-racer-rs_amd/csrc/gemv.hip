@@ -589,23 +589,50 @@ static hipError_t go_type(const GemvArgs &a, uint32_t act, hipStream_t s)
     }
 }
 
-// Batched K-quant rows above 16 tokens that the skinny kernel does not take
-// (more than 32 rows, Q6_K, K > 3072) run on the prefill GEMM's fp16 matrix
-// cores: the f32 rows become f16 block floating point (a power-of-two scale
-// per row, undone exactly on the output), zero-padded to a multiple of 128
-// rows inside the context workspace.
-static bool batched_gemm_route(const GemvArgs &a, uint32_t act)
+// Batched K-quant rows on the prefill GEMM's fp16 matrix cores: the f32 rows
+// become f16 block floating point (a power-of-two scale per row, undone
+// exactly on the output), zero-padded to a multiple of 128 rows inside the
+// context workspace.
+static bool batched_gemm_route(const GemvArgs &a)
 {
-    return a.M > 16 && act == ACT_PLAIN && !a.residual && a.type != T_F32 && a.ws &&
-           (((uintptr_t)a.x | (uintptr_t)a.y) & 15) == 0 && gemm_rows_supported(a.type, a.K, a.N, a.M, a.ws_bytes);
+    return a.M > 16 && !a.residual && a.type != T_F32 && a.ws && (((uintptr_t)a.x | (uintptr_t)a.y) & 15) == 0 &&
+           gemm_rows_supported(a.type, a.K, a.N, a.M, a.ws_bytes);
+}
+
+// M > 1 rows of plain activations.  2 to 4 rows: the int8 GEMV's multi-token
+// form where it applies (K <= 3072, 2 rows to 8192).  To 16 rows: the skinny
+// kernel with hi/lo activations, f32 accuracy.  17 to 32 rows: the skinny
+// kernel with f16 activations where such rows may be f16 (Q4_K / Q5_K with
+// K <= 3072, and what the GEMM takes); the GEMM above 32.  Where they may not
+// (N not a multiple of 64, unaligned rows), 16 rows at a time with hi/lo
+// activations.  Returns hipErrorNotSupported for what only the VALU kernels
+// take (F32 weights, tensors of 2 GB).
+static hipError_t launch_rows(const GemvArgs &a, hipStream_t s)
+{
+    if (gemv_mq_tokens_supported(a)) return launch_gemv_mq_tokens(a, s);
+    const bool gemm = batched_gemm_route(a);
+    if (skinny_supported(a) && (a.M <= 16 || gemm || (a.type != T_Q6_K && a.K <= 3072))) return launch_skinny(a, s);
+    if (gemm) return launch_gemm_f32_rows(a.x, a.W, a.type, a.y, a.K, a.N, a.M, a.ws, a.ws_bytes, s);
+    GemvArgs r = a;
+    r.M = a.M < 16 ? a.M : 16;
+    if (!skinny_supported(r)) return hipErrorNotSupported;
+    for (uint32_t m = 0; m < a.M; m += 16) {
+        r.M = a.M - m < 16 ? a.M - m : 16;
+        r.x = a.x + (uint64_t)m * a.K;
+        r.y = a.y + (uint64_t)m * a.N;
+        const hipError_t e = launch_skinny(r, s);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_gemv(const GemvArgs &a, uint32_t act, hipStream_t s)
 {
     if (gemv_mfma_supported(a)) return launch_gemv_mfma(a, act, s);
-    if (a.M > 1 && act == ACT_PLAIN && gemv_mq_tokens_supported(a)) return launch_gemv_mq_tokens(a, s);
-    if (a.M > 1 && act == ACT_PLAIN && skinny_supported(a)) return launch_skinny(a, s);
-    if (batched_gemm_route(a, act)) return launch_gemm_f32_rows(a.x, a.W, a.type, a.y, a.K, a.N, a.M, a.ws, a.ws_bytes, s);
+    if (a.M > 1 && act == ACT_PLAIN) {
+        const hipError_t e = launch_rows(a, s);
+        if (e != hipErrorNotSupported) return e;
+    }
     switch (a.type) {
     case T_Q4_K: return go_type<DecQ4K>(a, act, s);
     case T_Q5_K: return go_type<DecQ5K>(a, act, s);

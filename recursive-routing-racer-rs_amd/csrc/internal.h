@@ -67,7 +67,8 @@ hipError_t launch_gemv_mfma_stamped(const GemvArgs &a, uint32_t act, hipStream_t
 constexpr uint32_t MQ_TOKENS_MAX = 4;
 bool gemv_mq_tokens_supported(const GemvArgs &a);
 hipError_t launch_gemv_mq_tokens(const GemvArgs &a, hipStream_t s);
-// fp16-MFMA batched GEMV for 2 <= M <= 32, Q4_K / Q5_K (skinny.hip)
+// fp16-MFMA batched GEMV for 1 <= M <= 32 K-quant rows (skinny.hip): f32
+// accuracy to 16 rows, f16 activations above
 bool skinny_supported(const GemvArgs &a);
 hipError_t launch_skinny(const GemvArgs &a, hipStream_t s);
 // CUs of the current device (cached per device)

@@ -1,6 +1,7 @@
 // skinny.hip -- batched GEMV / skinny GEMM on the fp16 matrix cores for
-// 2 <= M <= 32 token rows and Q4_K / Q5_K weights (the batched shape of
-// phi4.rs:1257-1268: Y[m][n] = sum_k X[m][k] * W[n][k], X and Y f32 row-major).
+// 2 <= M <= 32 token rows and Q4_K / Q5_K / Q6_K weights of any K (the batched
+// shape of phi4.rs:1257-1268: Y[m][n] = sum_k X[m][k] * W[n][k], X and Y f32
+// row-major).
 //
 // Exact weights.  For super-block b of row n,
 //     sum_k x_k w_k = d * sum_s sum_{k in s} (sc_s q_k) x_k - dmin * sum_s mn_s X_s
@@ -22,28 +23,51 @@
 // k = 8(l/16) .. +7; 16x16x16 f16 -- the same at k = 4(l/16) .. +3; D rows
 // 4(l/16)+r of column l%16 in register r.
 //
-// Encoding pass (M > 8: two A tiles).  The A operands depend only on X, so a
-// small kernel (skinny_encode_kernel, one wave per A tile and super-block
-// column) builds them once per call into the workspace, in the lane order of
-// the MFMA:
-//   av   [TOK][W][8][64] f16x8  lane's 8 values of sub-block s
-//   amin [TOK][W][64]    f16x4  lane's 4 sub-block sums (min-term A operand)
-//   ex   [TOK][W][16]    int    E of A row r
-// (W = K/256 columns, TOK A tiles), 8,768 bytes per (tile, column).  Every
+// Encoding pass.  The A operands depend only on X, so a small kernel
+// (skinny_encode_kernel) builds them once per call into the workspace, in the
+// lane order of the MFMA:
+//   av   [TOK][B][8][64] f16x8  lane's 8 values of sub-block s
+//   amin [TOK][B][64]    f16x4  lane's 4 sub-block sums (min-term A operand)
+//   pe   [TOK][B][16]    f32    2^E of the A tile's token r (8 or 16 of them)
+// (B = K/256 columns, TOK A tiles), 8,768 bytes per (tile, column).  Every
 // workgroup of the main kernel then loads its operands with 16-byte loads
-// instead of reading all of X in f32 and converting it again.  With one A
-// tile (M <= 8) each wave encodes its own slice: there the pass's launch
-// costs more than the staging it saves (gate+up 16384x3072 at M = 4:
-// 16.5 us with it, 14.4 us without).
+// instead of reading all of X in f32 and converting it again: at 8 rows QKV
+// 5120x3072 takes 9.5 us against 10.1 with the operands built in every wave,
+// gate+up 16384x3072 13.8 against 14.5.
 //
-// Work split: a workgroup of K/256 waves, wave w owns super-block w of every
-// row; it gets its A operands (its first tiles' weight loads in flight), then
-// walks the workgroup's 16-row tiles b, b + G, ... (G = gridDim.x), staging the
-// tile's 16 blocks of its column in its private LDS region by LDS DMA (the
-// next tiles' loads in flight meanwhile).  Row partials of the waves are added
-// in wave order per tile.
+// Work split: a workgroup of W waves takes the 16-row tiles b, b + G, ... (G =
+// gridDim.x), T of them at a time; wave w owns the super-block columns w,
+// w + W, ... of every row.  It walks its columns: the column's A operands in
+// registers (the next column's requested meanwhile), then the T tiles' 16
+// blocks of that column, staged in the wave's private LDS ring by LDS DMA (the
+// next units in flight).  The row sums of the T tiles stay in registers over
+// all columns; one barrier per T tiles, then the waves' partials are added in
+// wave order.
+//
+// Q6_K.  p = sc_s (q - 32) reaches 127 * 32 = 4064, 13 bits with sign: one
+// fp16 holds it up to 2048, above that to the next even number.  B hi =
+// fp16(p) and B lo = p - B hi (exact, one packed fma) are two MFMAs on the same
+// A operand, so the weight stays exact at the hi/lo activations; with hi
+// activations alone (M > 16) B hi is taken alone, its 2^-12 is that bar's.
+// A 210-byte block starts 2 bytes past a dword when its index is odd: rows are
+// loaded from the dword below (14 units of 16 bytes a row) and moved down 2
+// bytes in registers (v_alignbyte).
+//
+// Bound: HBM at every M in principle (20.6 MB of Q6_K in 2.9 us); in fact a CU's
+// intake (at K = 8192 and 8 rows 262 KB of A operands next to its 80 KB of
+// weights) and the decode (~330 VALU instructions a unit, three waves a SIMD).
+// Measured per call, graphs over 300 MB of weight copies, in us, against the
+// VALU kernel (four rows a pass over the weights) and, at 27 rows, the row
+// conversion + prefill GEMM + split reduction that took these shapes before:
+//   3072x8192 Q6_K  8 rows 16.3 (69), 16 rows 19.5 (134), 27 rows 19.6 (29.7)
+//   3072x8192 Q4_K  8 rows 14.2 (39), 16 rows 17.2 (71),  27 rows 18.0 (25.8)
+// and against the form with one column a wave and a barrier per tile:
+//   16384x3072 Q4_K 8 rows 13.8 (15.6), 27 rows 16.2 (18.3)
+//   5120x3072 Q5_K  8 rows 9.5 (11.0),  27 rows 11.2 (12.4)
 #include "device_common.h"
 #include "internal.h"
+
+#include <type_traits>
 
 namespace rrr {
 
@@ -51,8 +75,8 @@ typedef _Float16 f16x8s __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4s __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x2s __attribute__((ext_vector_type(2)));
 
-// Scalar offset past every weight byte (w_bytes + RRR_READ_SLACK must stay
-// below it): such loads return zeros and move no data.
+// Lane offset past every weight byte (w_bytes + RRR_READ_SLACK must stay below
+// it): such loads return zeros and move no data.
 constexpr uint32_t SK_OOB = 0x80000000u;
 
 __device__ __forceinline__ f16x2s sk_bits(uint32_t v) { return __builtin_bit_cast(f16x2s, v); }
@@ -70,9 +94,10 @@ __device__ __forceinline__ void sk_scale4(uint32_t v, f16x2s sc2, f16x2s nb2, ui
 // Q4_K (phi4.rs:481-510): element 32s + e of a block is nibble (s & 1) of
 // qs[32 (s/2) + e].  Lane k-group kg takes e = 8kg .. 8kg+7 of every s.
 struct SkQ4K {
-    static constexpr uint32_t BS = 144;
+    static constexpr uint32_t BS = 144, LROW = 144;   // bytes of a block, and of its row in LDS
+    static constexpr bool MINS = true;                // a min term (d*sc*q - dmin*mn)
     struct Raw { u32x4 hdr; u32x2 qs[4]; };
-    __device__ static void load(Raw &r, const uint8_t *L, uint32_t o, uint32_t kg)
+    __device__ static void load(Raw &r, const uint8_t *L, uint32_t o, uint32_t kg, uint32_t)
     {
         r.hdr = *(const u32x4 *)(L + o);
 #pragma unroll
@@ -88,9 +113,10 @@ struct SkQ4K {
 
 // Q5_K (phi4.rs:512-542): Q4_K's nibbles plus bit s of qh[e] as bit 4.
 struct SkQ5K {
-    static constexpr uint32_t BS = 176;
+    static constexpr uint32_t BS = 176, LROW = 176;
+    static constexpr bool MINS = true;
     struct Raw { u32x4 hdr; u32x2 qh; u32x2 qs[4]; };
-    __device__ static void load(Raw &r, const uint8_t *L, uint32_t o, uint32_t kg)
+    __device__ static void load(Raw &r, const uint8_t *L, uint32_t o, uint32_t kg, uint32_t)
     {
         r.hdr = *(const u32x4 *)(L + o);
         r.qh = *(const u32x2 *)(L + o + 16 + 8 * kg);
@@ -104,6 +130,58 @@ struct SkQ5K {
     }
 };
 
+// Q6_K (phi4.rs:444-479): element 32s + e of a block is nibble (s % 4) / 2 of
+// ql[64 (s/4) + 32 (s & 1) + e] and bits 2 (s % 4) .. +1 of qh[32 (s/4) + e],
+// minus 32, times sc[2s + e/16].  The block starts `odd` (0 or 2) bytes into
+// its LDS row.
+struct SkQ6K {
+    static constexpr uint32_t BS = 210, LROW = 224;
+    static constexpr bool MINS = false;
+    struct Raw { u32x2 ql[4], qh[2]; uint32_t sc[4]; uint32_t d; };
+    // 8 bytes at p + odd, p 8-byte aligned
+    __device__ static u32x2 at(const uint8_t *p, uint32_t odd)
+    {
+        const u32x2 v = *(const u32x2 *)p;
+        const uint32_t n = *(const uint32_t *)(p + 8);
+        return u32x2{__builtin_amdgcn_alignbyte(v.y, v.x, odd), __builtin_amdgcn_alignbyte(n, v.y, odd)};
+    }
+    __device__ static void load(Raw &r, const uint8_t *L, uint32_t o, uint32_t kg, uint32_t odd)
+    {
+        const uint8_t *p = L + o;
+#pragma unroll
+        for (int i = 0; i < 4; i++) r.ql[i] = at(p + 32 * i + 8 * kg, odd);
+#pragma unroll
+        for (int i = 0; i < 2; i++) r.qh[i] = at(p + 128 + 32 * i + 8 * kg, odd);
+        const u32x4 c = *(const u32x4 *)(p + 192);
+        const uint32_t e = *(const uint32_t *)(p + 208);
+        r.sc[0] = __builtin_amdgcn_alignbyte(c.y, c.x, odd);
+        r.sc[1] = __builtin_amdgcn_alignbyte(c.z, c.y, odd);
+        r.sc[2] = __builtin_amdgcn_alignbyte(c.w, c.z, odd);
+        r.sc[3] = __builtin_amdgcn_alignbyte(e, c.w, odd);
+        r.d = e >> (8 * odd);
+    }
+    __device__ static void quants(const Raw &r, int s, uint32_t &v0, uint32_t &v1)
+    {
+        const int g = s >> 2, q = s & 3;
+        const u32x2 l = r.ql[2 * g + (q & 1)], h = r.qh[g];
+        v0 = ((l.x >> (4 * (q >> 1))) & 0x0F0F0F0Fu) | (((h.x >> (2 * q)) & 0x03030303u) << 4);
+        v1 = ((l.y >> (4 * (q >> 1))) & 0x0F0F0F0Fu) | (((h.y >> (2 * q)) & 0x03030303u) << 4);
+    }
+};
+
+// Four quant values (bytes < 64 of v) minus 32, times the scale, as fp16 hi + lo.
+__device__ __forceinline__ void sk_scale4_q6(uint32_t v, f16x2s sc2, uint32_t (&hi)[2], uint32_t (&lo)[2])
+{
+    const f16x2s off = {(_Float16)1056.0f, (_Float16)1056.0f};
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const f16x2s q = sk_bits(__builtin_amdgcn_perm(0x64646464u, v, i ? 0x04030402u : 0x04010400u)) - off;
+        const f16x2s h = q * sc2;
+        hi[i] = sk_u32(h);
+        lo[i] = sk_u32(__builtin_elementwise_fma(q, sc2, -h));
+    }
+}
+
 // Staging geometry of one wave's 16 block pieces, loaded straight into LDS
 // (16-byte LDS DMA: lane l of a load writes base + 16 l).  Load slot s covers
 // rows s*RPS .. s*RPS+RPS-1 (lane l: unit l % UPB of row l / UPB) and has a
@@ -111,327 +189,409 @@ struct SkQ5K {
 // and write zeros) stay inside it.  A tile buffer is S slots.
 template <class Q>
 struct SkGeom {
-    static constexpr uint32_t UPB = Q::BS / 16;
+    static constexpr uint32_t UPB = Q::LROW / 16;
     static constexpr uint32_t RPS = 64 / UPB;
     static constexpr int S = (16 + RPS - 1) / RPS;
     static constexpr uint32_t BUF = 1024 * S;
     // LDS offset of row r inside a tile buffer
-    __device__ static uint32_t row_off(uint32_t r) { return (r / RPS) * 1024 + (r % RPS) * Q::BS; }
+    __device__ static uint32_t row_off(uint32_t r) { return (r / RPS) * 1024 + (r % RPS) * Q::LROW; }
 };
 
 // Workspace layout of the encoded activations (see the top of this file).
-constexpr uint32_t SK_AV_UNIT = 8 * 64 * 16, SK_AMIN_UNIT = 64 * 8, SK_EX_UNIT = 16 * 4;
-__host__ __device__ constexpr uint64_t sk_ws_bytes(uint32_t tok, uint32_t W)
+constexpr uint32_t SK_AV_UNIT = 8 * 64 * 16, SK_AMIN_UNIT = 64 * 8, SK_PE_UNIT = 16 * 4;
+__host__ __device__ constexpr uint64_t sk_ws_bytes(uint32_t tok, uint32_t B)
 {
-    return (uint64_t)tok * W * (SK_AV_UNIT + SK_AMIN_UNIT + SK_EX_UNIT);
+    return (uint64_t)tok * B * (SK_AV_UNIT + SK_AMIN_UNIT + SK_PE_UNIT);
 }
 struct SkWs {
-    u32x4 *av;
-    u32x2 *amin;
-    int *ex;
-    __host__ __device__ SkWs(void *base, uint32_t tok, uint32_t W)
+    uint32_t amin, pe, bytes;   // byte offsets of the parts (av at 0), and the end
+    __host__ __device__ SkWs(uint32_t tok, uint32_t B)
+        : amin(tok * B * SK_AV_UNIT), pe(amin + tok * B * SK_AMIN_UNIT), bytes(pe + tok * B * SK_PE_UNIT)
     {
-        uint8_t *p = (uint8_t *)base;
-        av = (u32x4 *)p;
-        amin = (u32x2 *)(p + (uint64_t)tok * W * SK_AV_UNIT);
-        ex = (int *)(p + (uint64_t)tok * W * (SK_AV_UNIT + SK_AMIN_UNIT));
     }
 };
 
-// A operands of A tile tt and super-block column w, built by one wave:
-// lane (row r16, group kg) gets token tok's values k0 + 32 s + 8 kg + i
-// (i < 8) of every sub-block s, its 4 sub-block sums (min-term A operand) and
-// the block exponent E of its A row.  HILO: 8 tokens (hi, lo rows) per A
-// tile, else 16 tokens (hi rows).  after_loads() runs once the activation
-// loads are issued (the caller queues its weight loads behind them).
-template <bool HILO, class F>
-__device__ __forceinline__ void sk_encode(const float *__restrict__ x, uint32_t M, uint32_t K, uint32_t tt,
-                                          uint32_t w, uint32_t lane, f16x8s (&av)[8], f16x4s &am, int &e,
-                                          F &&after_loads)
+// max |.| and sum of 8 values
+__device__ __forceinline__ float sk_max8(const float4 &u, const float4 &v)
 {
+    return fmaxf(fmaxf(fmaxf(fabsf(u.x), fabsf(u.y)), fmaxf(fabsf(u.z), fabsf(u.w))),
+                 fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+}
+__device__ __forceinline__ float sk_sum8(const float4 &u, const float4 &v)
+{
+    return ((u.x + u.y) + (u.z + u.w)) + ((v.x + v.y) + (v.z + v.w));
+}
+// E of a slice whose largest |x| is mx: mx / 2^E in [2^13, 2^14)
+__device__ __forceinline__ int sk_exponent(float mx)
+{
+    int ex = 14;
+    if (mx > 0.0f && __builtin_isfinite(mx)) (void)frexpf(mx, &ex);
+    return ex - 14;
+}
+// v / 2^e in f16: its hi or lo half (ldexp: times 2^-e would overflow for a
+// slice below 2^-113), 0 for a row past M
+__device__ __forceinline__ _Float16 sk_half(float v, int e, bool lo, bool live)
+{
+    const float y = ldexpf(v, -e);
+    const _Float16 hi = (_Float16)y;
+    return live ? (lo ? (_Float16)(y - (float)hi) : hi) : (_Float16)0.0f;
+}
+__device__ __forceinline__ f16x8s sk_values(const float4 &u, const float4 &v, int e, bool lo, bool live)
+{
+    const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+    f16x8s h;
+#pragma unroll
+    for (int i = 0; i < 8; i++) h[i] = sk_half(f[i], e, lo, live);
+    return h;
+}
+
+// The encoding pass: one workgroup of four waves per (super-block column, A
+// tile), grid (B, TOK).  Lane (row r16, group kg) of wave q takes token tok's
+// values 32 s + 8 kg + i (i < 8) of sub-blocks s = 2q, 2q + 1.  Bound by latency
+// (a load, a maximum over the slice, a store): one wave for all eight sub-blocks
+// was a chain of ~600 instructions (with this split QKV 5120x3072 at 16 rows
+// went from 12.1 to 11.2 us a call).  HILO: 8 tokens (hi, lo rows) per A tile,
+// else 16 tokens (hi rows).
+template <bool HILO>
+__global__ __launch_bounds__(256) void skinny_encode_kernel(const float *__restrict__ x, uint32_t M, uint32_t K,
+                                                            uint8_t *ws, uint32_t tok_tiles)
+{
+    __shared__ float wmax[4][16], gsum[8][16];
+    const uint32_t B = K / 256, c = blockIdx.x, tt = blockIdx.y, lane = threadIdx.x & 63, q = threadIdx.x >> 6;
     const uint32_t r16 = lane & 15, kg = lane >> 4;
-    const uint32_t k0 = w * 256;
+    const SkWs o(tok_tiles, B);
     const uint32_t tok = HILO ? tt * 8 + (r16 >> 1) : tt * 16 + r16;
     const bool lo = HILO && (r16 & 1);
     const bool live = tok < M;
-    const float4 *xp = (const float4 *)(x + (uint64_t)min(tok, M - 1) * K + k0 + 8 * kg);
-    float4 xv[16];
+    const float4 *xp = (const float4 *)(x + (uint64_t)min(tok, M - 1) * K + c * 256 + 64 * q + 8 * kg);
+    const float4 xv[4] = {xp[0], xp[1], xp[8], xp[9]};
+    float mx = 0.0f, gs[2];
 #pragma unroll
-    for (int s = 0; s < 8; s++) {
-        xv[2 * s] = xp[8 * s];
-        xv[2 * s + 1] = xp[8 * s + 1];
-    }
-    after_loads();
-    float mx = 0.0f, gs[8];
-#pragma unroll
-    for (int s = 0; s < 8; s++) {
+    for (int s = 0; s < 2; s++) {
         const float4 u = xv[2 * s], v = xv[2 * s + 1];
-        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(u.x), fabsf(u.y)), fmaxf(fabsf(u.z), fabsf(u.w))));
-        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-        gs[s] = ((u.x + u.y) + (u.z + u.w)) + ((v.x + v.y) + (v.z + v.w));
+        mx = fmaxf(mx, sk_max8(u, v));
+        gs[s] = sk_sum8(u, v);
     }
-    // the token's four k-groups (lanes r16 + 16 kg)
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
 #pragma unroll
-    for (int s = 0; s < 8; s++) {
+    for (int s = 0; s < 2; s++) {
         gs[s] = gs[s] + __shfl_xor(gs[s], 16, 64);
         gs[s] = gs[s] + __shfl_xor(gs[s], 32, 64);
     }
-    e = 0;
-    if (mx > 0.0f && __builtin_isfinite(mx)) {
-        int ex;
-        (void)frexpf(mx, &ex);
-        e = ex - 14;  // mx / 2^e in [2^13, 2^14)
+    if (kg == 0) {
+        wmax[q][r16] = mx;
+        gsum[2 * q][r16] = gs[0];
+        gsum[2 * q + 1][r16] = gs[1];
     }
-    const float sx = ldexpf(1.0f, -e), sg = ldexpf(1.0f, -e - 5);
+    __syncthreads();
+    const int e = sk_exponent(fmaxf(fmaxf(wmax[0][r16], wmax[1][r16]), fmaxf(wmax[2][r16], wmax[3][r16])));
+    u32x4 *ap = (u32x4 *)ws + (uint64_t)(tt * B + c) * 8 * 64 + lane;
 #pragma unroll
-    for (int s = 0; s < 8; s++) {
-        const float4 u = xv[2 * s], v = xv[2 * s + 1];
-        const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-        f16x8s h;
+    for (int s = 0; s < 2; s++)
+        ap[(2 * q + s) * 64] = __builtin_bit_cast(u32x4, sk_values(xv[2 * s], xv[2 * s + 1], e, lo, live));
+    if (q != 0) return;
+    f16x4s am;
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float y = f[i] * sx;
-            const _Float16 hi = (_Float16)y;
-            h[i] = live ? (lo ? (_Float16)(y - (float)hi) : hi) : (_Float16)0.0f;
-        }
-        av[s] = h;
-    }
-    // X_s of sub-blocks 4 kg .. 4 kg + 3 (k-groups 2, 3 are padding)
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        float g = 0.0f;
-#pragma unroll
-        for (int s = 0; s < 8; s++)
-            if (s == (int)(4 * kg) + i) g = gs[s];
-        const float y = g * sg;
-        const _Float16 hi = (_Float16)y;
-        am[i] = live && kg < 2 ? (lo ? (_Float16)(y - (float)hi) : hi) : (_Float16)0.0f;
-    }
+    for (int i = 0; i < 4; i++) am[i] = sk_half(gsum[(4 * kg + i) & 7][r16], e + 5, lo, live && kg < 2);
+    ((u32x2 *)(ws + o.amin))[(uint64_t)(tt * B + c) * 64 + lane] = __builtin_bit_cast(u32x2, am);
+    // lanes 0..15 hold A rows 0..15: rows 2t, 2t + 1 (HILO) or row t are token t
+    if (lane < 16 && (!HILO || !(lane & 1)))
+        ((float *)(ws + o.pe))[(tt * B + c) * 16 + (HILO ? lane >> 1 : lane)] = ldexpf(1.0f, e);
 }
 
-// The encoding pass: one wave per (super-block column, A tile), grid (W, TOK).
-template <bool HILO>
-__global__ __launch_bounds__(64) void skinny_encode_kernel(const float *__restrict__ x, uint32_t M, uint32_t K,
-                                                           void *ws, uint32_t tok_tiles)
+// The A operands of one super-block column: TOK A tiles, pe the 2^E of the
+// lane's D-layout tokens (D row 4 kg + j holds A row 4 kg + j: HILO token
+// 2 kg + j / 2, else token 4 kg + j).
+template <int TOK, int DPT>
+struct SkA {
+    f16x8s av[TOK][8];
+    f16x4s amin[TOK];
+    float pe[TOK][DPT];
+};
+
+// Tile buffers a wave of a WMAX-wave workgroup gets out of the 160 KB of LDS.
+template <class Q, int WMAX>
+constexpr int sk_ring()
 {
-    const uint32_t W = K / 256, w = blockIdx.x, tt = blockIdx.y, lane = threadIdx.x;
-    const SkWs o(ws, tok_tiles, W);
-    f16x8s av[8];
-    f16x4s am;
-    int e;
-    sk_encode<HILO>(x, M, K, tt, w, lane, av, am, e, [] {});
-    u32x4 *ap = o.av + (uint64_t)(tt * W + w) * 8 * 64 + lane;
-#pragma unroll
-    for (int s = 0; s < 8; s++) ap[s * 64] = __builtin_bit_cast(u32x4, av[s]);
-    o.amin[(uint64_t)(tt * W + w) * 64 + lane] = __builtin_bit_cast(u32x2, am);
-    if (lane < 16) o.ex[(tt * W + w) * 16 + lane] = e;
+    constexpr int n = 160 * 1024 / (WMAX * (int)SkGeom<Q>::BUF);
+    return n > 4 ? 4 : n;
 }
 
 // TOK A tiles (TPT tokens each); DPT = tokens of a tile per lane in the D
-// layout.  NB tile buffers per wave: tiles i+1 .. i+NB-1 stream in while
-// tile i is multiplied.  PRE: the A operands come from the encoding pass,
-// else each wave builds its own (one A tile: the f32 activations are no more
-// bytes than their encoding, and the pass would cost a launch).
-template <class Q, bool HILO, int TOK, int NB, bool PRE>
-__global__ __launch_bounds__(TOK == 1 ? 1024 : 768) void skinny_kernel(GemvArgs a, uint32_t ntiles)
+// layout; T tiles at a time.  At most WMAX waves, NB = sk_ring tile buffers
+// per wave: units u + 1 .. u + NB - 1 stream in while unit u is multiplied
+// (unit = column, tile).  DB: more than one column a wave, the next column's A
+// operands requested one column ahead.
+template <class Q, bool HILO, int TOK, int T, int WMAX, bool DB>
+__global__ __launch_bounds__(64 * WMAX) void skinny_kernel(GemvArgs a, uint32_t ntiles)
 {
     using G = SkGeom<Q>;
-    constexpr int TPT = HILO ? 8 : 16, DPT = HILO ? 2 : 4, MP = TOK * TPT;
+    constexpr int TPT = HILO ? 8 : 16, DPT = HILO ? 2 : 4, MP = TOK * TPT, NB = sk_ring<Q, WMAX>();
+    constexpr int NA = DB ? TOK * (9 + (Q::MINS ? 1 : 0)) : 0;   // loads of one column's A operands
+    constexpr int AHEAD = DB || NB - 1 < T ? NB - 1 : T;         // units issued before the first
+    static_assert(NB >= 2 && NB * G::BUF >= (uint32_t)T * MP * 64, "ring: two units, and the wave's row sums");
     extern __shared__ float smem[];
-    const uint32_t K = a.K, M = a.M, N = a.N, W = K / 256;
+    const uint32_t K = a.K, M = a.M, N = a.N, B = K / 256, W = blockDim.x / 64;
     const uint32_t t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const uint32_t r16 = lane & 15, kg = lane >> 4;
     const uint32_t GR = gridDim.x, tile0 = blockIdx.x;
-    const uint32_t ntl = tile0 < ntiles ? (ntiles - tile0 + GR - 1) / GR : 0u;
-    uint8_t *L = (uint8_t *)smem + wave * NB * G::BUF;            // this wave's tile buffers
-    float *part = (float *)((uint8_t *)smem + W * NB * G::BUF);  // [2][W][MP][16]
+    const uint32_t Cw = (B - wave + W - 1) / W;          // this wave's columns wave, wave + W, ... (W <= B)
+    uint8_t *L = (uint8_t *)smem + wave * NB * G::BUF;   // this wave's tile buffers, then its row sums
 
-    const uint32_t row_bytes = W * Q::BS;
+    const uint32_t row_bytes = B * Q::BS;
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.W, a.w_bytes + RRR_READ_SLACK);
 
     // weight units: lane-fixed offsets, a uniform offset per load slot; rows
     // past 16 in the last slot read nothing
     const uint32_t rsel = min(lane / G::UPB, G::RPS - 1), vl = lane - (lane / G::UPB) * G::UPB;
     const bool lane_ok = lane < G::RPS * G::UPB;
-    const uint32_t voff = lane_ok ? rsel * row_bytes + wave * Q::BS + 16 * vl : SK_OOB;
-    const uint32_t voff_last = (G::S - 1) * G::RPS + rsel < 16 ? voff : SK_OOB;
+    const bool last_ok = lane_ok && (G::S - 1) * G::RPS + rsel < 16;
     const uint32_t tile_bytes = 16 * row_bytes;
-    // tile tl into buffer tl % NB (S loads; past the last tile: zeros)
-    auto dma = [&](uint32_t tl) {
-        const uint32_t tb = tl < ntl ? (tile0 + tl * GR) * tile_bytes : SK_OOB;
-        uint8_t *dst = L + (tl % NB) * G::BUF;
+    // tile `tile` of the wave's column ci into buffer `buf` (S loads; past the
+    // last tile or column: zeros).  Q6_K: an odd block from the dword below (a
+    // tile's and a slot's first rows have even block numbers, as S * RPS = 16
+    // and RPS = 4 rows)
+    auto dma = [&](uint32_t ci, uint32_t tile, uint32_t buf) {
+        const uint32_t c = wave + ci * W;
+        const uint32_t odd = Q::MINS ? 0u : 2 * ((rsel * B + c) & 1);
+        const uint32_t v = rsel * row_bytes + c * Q::BS - odd + 16 * vl;
+        const bool live = ci < Cw && tile < ntiles;
+        const uint32_t tb = live ? tile * tile_bytes : 0u;
+        uint8_t *dst = L + buf * G::BUF;
 #pragma unroll
         for (int s = 0; s < G::S; s++)
-            lds_dma16<RRR_CPOL_NT>(rs, dst + 1024 * s, s == G::S - 1 ? voff_last : voff, tb + s * G::RPS * row_bytes);
+            lds_dma16<RRR_CPOL_NT>(rs, dst + 1024 * s, live && (s == G::S - 1 ? last_ok : lane_ok) ? v : SK_OOB,
+                                   tb + s * G::RPS * row_bytes);
     };
 
-    // 1. A operands, the first tiles' weights streaming in meanwhile (queued
-    // after the loads of the encoded operands, and after those of f32
-    // activations, which the encoding needs first: loads return in order, so
-    // tile 0 waits for the A operands and its own weights only, while the
-    // next tiles' weights arrive under its MFMAs)
-    f16x8s av[TOK][8];
-    f16x4s amin[TOK];
-    int eexp[TOK][DPT];   // E of the lane's D-layout tokens
-    // D row 4 kg + j holds A row 4 kg + j: the token of A row 4 kg + 2 j
-    // (HILO: rows 2t, 2t+1 are token t's hi and lo) or 4 kg + j
-    if constexpr (PRE) {
-        const SkWs o(a.ws, TOK, W);
+    // A operands of the wave's column ci from the encoding pass (NA loads;
+    // past the last column: no request)
+    using A = SkA<TOK, DPT>;
+    const SkWs o(TOK, B);
+    const __amdgpu_buffer_rsrc_t ra = make_rsrc(a.ws, o.bytes);
+    auto load_a = [&](A &x, uint32_t ci) {
+        const uint32_t out = ci < Cw ? 0u : RRR_OOB, c = wave + ci * W;
 #pragma unroll
         for (int tt = 0; tt < TOK; tt++) {
-            const u32x4 *ap = o.av + (uint64_t)(tt * W + wave) * 8 * 64 + lane;
+            const uint32_t u = tt * B + (ci < Cw ? c : 0u);
 #pragma unroll
-            for (int s = 0; s < 8; s++) av[tt][s] = __builtin_bit_cast(f16x8s, ap[s * 64]);
-            amin[tt] = __builtin_bit_cast(f16x4s, o.amin[(uint64_t)(tt * W + wave) * 64 + lane]);
-#pragma unroll
-            for (int j = 0; j < DPT; j++)
-                eexp[tt][j] = o.ex[(tt * W + wave) * 16 + (HILO ? 4 * kg + 2 * j : 4 * kg + j)];
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        for (uint32_t i = 0; i + 1 < NB; i++) dma(i);
-    } else {
-#pragma unroll
-        for (int tt = 0; tt < TOK; tt++) {
-            int e;
-            sk_encode<HILO>(a.x, M, K, tt, wave, lane, av[tt], amin[tt], e, [&] {
-                if (tt == 0)
-                    for (uint32_t i = 0; i + 1 < NB; i++) dma(i);
-            });
-#pragma unroll
-            for (int j = 0; j < DPT; j++) eexp[tt][j] = __shfl(e, HILO ? 4 * kg + 2 * j : 4 * kg + j, 64);
-        }
-    }
-
-    // 2^E of the lane's D-layout tokens (the same for every tile)
-    float pe[TOK][DPT];
-#pragma unroll
-    for (int tt = 0; tt < TOK; tt++)
-#pragma unroll
-        for (int j = 0; j < DPT; j++) pe[tt][j] = ldexpf(1.0f, eexp[tt][j]);
-    // 2. tiles: tile tl + NB - 1 into the buffer tile tl - 1 used, wait for
-    // tile tl, MFMAs, row partials
-    uint32_t buf = 0;
-    const uint32_t roff = G::row_off(r16);
-    for (uint32_t tl = 0; tl < ntl; tl++) {
-        dma(tl + NB - 1);
-        wait_vm<(NB - 1) * G::S>();
-        typename Q::Raw raw;
-        Q::load(raw, L + (tl % NB) * G::BUF, roff, kg);
-        const float d = h2f(raw.hdr.x), dmin = h2f(raw.hdr.x >> 16);
-        uint32_t scb[2], mnb[2];
-        scale_min_bytes_k4(raw.hdr.y, raw.hdr.z, raw.hdr.w, scb, mnb);
-        // min term B operand: mn of sub-blocks 4 kg .. 4 kg + 3 (k-groups 2, 3 padding)
-        const uint32_t mk = kg == 0 ? mnb[0] : mnb[1];
-        const f16x2s m01 = sk_bits(__builtin_amdgcn_perm(0x64646464u, mk, 0x04010400u)) - f16x2s{(_Float16)1024.0f, (_Float16)1024.0f};
-        const f16x2s m23 = sk_bits(__builtin_amdgcn_perm(0x64646464u, mk, 0x04030402u)) - f16x2s{(_Float16)1024.0f, (_Float16)1024.0f};
-        const f16x4s bmin = kg < 2 ? f16x4s{m01[0], m01[1], m23[0], m23[1]} : f16x4s{(_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f};
-        f32x4 acc[TOK], accm[TOK];
-#pragma unroll
-        for (int tt = 0; tt < TOK; tt++) acc[tt] = accm[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < 8; s++) {
-            // {sc_s, sc_s} exactly: byte s under the exponent of 1024, minus 1024
-            const f16x2s sc2 = sk_bits(__builtin_amdgcn_perm(0x64646464u, scb[s >> 2], 0x04000400u + 0x00010001u * (s & 3))) -
-                               f16x2s{(_Float16)1024.0f, (_Float16)1024.0f};
-            const f16x2s nb2 = sc2 * f16x2s{(_Float16)-1024.0f, (_Float16)-1024.0f};
-            uint32_t v0, v1, b[4];
-            Q::quants(raw, s, v0, v1);
-            sk_scale4(v0, sc2, nb2, b[0], b[1]);
-            sk_scale4(v1, sc2, nb2, b[2], b[3]);
-            const f16x8s bv = __builtin_bit_cast(f16x8s, u32x4{b[0], b[1], b[2], b[3]});
-#pragma unroll
-            for (int tt = 0; tt < TOK; tt++) acc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[tt][s], bv, acc[tt], 0, 0, 0);
-            // one sub-block's B operand live at a time
-            if constexpr (TOK > 1) __builtin_amdgcn_sched_barrier(0);
-        }
-        // the row partials of this wave: d * 2^E * S - dmin * 2^(E+5) * S_min
-        float *pp = part + (size_t)buf * W * MP * 16 + (size_t)wave * MP * 16 + r16;
-#pragma unroll
-        for (int tt = 0; tt < TOK; tt++) {
-            accm[tt] = __builtin_amdgcn_mfma_f32_16x16x16f16(amin[tt], bmin, accm[tt], 0, 0, 0);
-#pragma unroll
-            for (int j = 0; j < DPT; j++) {
-                const float sv = HILO ? acc[tt][2 * j] + acc[tt][2 * j + 1] : acc[tt][j];
-                const float sm = HILO ? accm[tt][2 * j] + accm[tt][2 * j + 1] : accm[tt][j];
-                const float v = pe[tt][j] * fmaf(d, sv, -(32.0f * dmin) * sm);
-                const uint32_t tok = tt * TPT + (HILO ? 2 * kg + j : 4 * kg + j);
-                pp[tok * 16] = v;
+            for (int s = 0; s < 8; s++)
+                x.av[tt][s] = __builtin_bit_cast(f16x8s, bload16_so(ra, (lane * 16 + s * 1024) | out, u * SK_AV_UNIT));
+            if constexpr (Q::MINS)
+                x.amin[tt] = __builtin_bit_cast(
+                    f16x4s, __builtin_amdgcn_raw_buffer_load_b64(ra, (lane * 8) | out, o.amin + u * SK_AMIN_UNIT, 0));
+            const uint32_t po = o.pe + u * SK_PE_UNIT;
+            if constexpr (HILO) {
+                const u32x2 p = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(ra, (8 * kg) | out, po, 0));
+                x.pe[tt][0] = u2f(p.x);
+                x.pe[tt][1] = u2f(p.y);
+            } else {
+                const u32x4 p = bload16_so(ra, (16 * kg) | out, po);
+                x.pe[tt][0] = u2f(p.x);
+                x.pe[tt][1] = u2f(p.y);
+                x.pe[tt][DPT - 2] = u2f(p.z);
+                x.pe[tt][DPT - 1] = u2f(p.w);
             }
         }
+    };
+
+    const uint32_t roff = G::row_off(r16);
+    float tot[T][TOK][DPT];   // row sums of the T tiles over the wave's columns
+    uint32_t buf = 0, tb0 = tile0;   // ring place of the next unit; the first of the T tiles
+
+    // one unit: tile ti of the T (static), the column's A operands in x
+    auto unit = [&](const A &x, uint32_t ci, auto tic) {
+        constexpr int ti = decltype(tic)::value;
+        // the unit NB - 1 ahead into the buffer the last unit left, once its
+        // LDS reads are done (a DMA that is out of range writes its zeros at once)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        // (one column a wave: none past its T tiles)
+        const uint32_t ahead = buf == 0 ? NB - 1 : buf - 1;
+        if constexpr (DB || ti + NB - 1 < T) dma(ci + (ti + NB - 1) / T, tb0 + ((ti + NB - 1) % T) * GR, ahead);
+        // this unit landed: issued before the next column's A operands if it
+        // is one of the column's first NB - 1, after them otherwise
+        constexpr int later = DB || ti + NB - 1 < T ? NB - 1 : T - 1 - ti;   // units issued after it
+        constexpr int n = later * G::S + (ti <= NB - 2 ? NA : 0);
+        wait_vm<(n < 63 ? n : 63)>();
+        typename Q::Raw raw;
+        const uint32_t odd = Q::MINS ? 0u : 2 * ((r16 * B + wave + ci * W) & 1);
+        Q::load(raw, L + buf * G::BUF, roff, kg, odd);
+        buf = buf + 1 == NB ? 0 : buf + 1;
+        f32x4 acc[TOK];
+#pragma unroll
+        for (int tt = 0; tt < TOK; tt++) acc[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const f16x2s k1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
+        if constexpr (Q::MINS) {
+            const float d = h2f(raw.hdr.x), dmin = h2f(raw.hdr.x >> 16);
+            uint32_t scb[2], mnb[2];
+            scale_min_bytes_k4(raw.hdr.y, raw.hdr.z, raw.hdr.w, scb, mnb);
+            // min term B operand: mn of sub-blocks 4 kg .. 4 kg + 3 (k-groups 2, 3 padding)
+            const uint32_t mk = kg == 0 ? mnb[0] : mnb[1];
+            const f16x2s m01 = sk_bits(__builtin_amdgcn_perm(0x64646464u, mk, 0x04010400u)) - k1024;
+            const f16x2s m23 = sk_bits(__builtin_amdgcn_perm(0x64646464u, mk, 0x04030402u)) - k1024;
+            const f16x4s bmin = kg < 2 ? f16x4s{m01[0], m01[1], m23[0], m23[1]} : f16x4s{(_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f};
+#pragma unroll
+            for (int s = 0; s < 8; s++) {
+                // {sc_s, sc_s} exactly: byte s under the exponent of 1024, minus 1024
+                const f16x2s sc2 = sk_bits(__builtin_amdgcn_perm(0x64646464u, scb[s >> 2], 0x04000400u + 0x00010001u * (s & 3))) - k1024;
+                const f16x2s nb2 = sc2 * -k1024;
+                uint32_t v0, v1, b[4];
+                Q::quants(raw, s, v0, v1);
+                sk_scale4(v0, sc2, nb2, b[0], b[1]);
+                sk_scale4(v1, sc2, nb2, b[2], b[3]);
+                const f16x8s bv = __builtin_bit_cast(f16x8s, u32x4{b[0], b[1], b[2], b[3]});
+#pragma unroll
+                for (int tt = 0; tt < TOK; tt++) acc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.av[tt][s], bv, acc[tt], 0, 0, 0);
+                // one sub-block's B operand live at a time
+                if constexpr (TOK > 1) __builtin_amdgcn_sched_barrier(0);
+            }
+            // the row partials: d * 2^E * S - dmin * 2^(E+5) * S_min
+#pragma unroll
+            for (int tt = 0; tt < TOK; tt++) {
+                const f32x4 accm = __builtin_amdgcn_mfma_f32_16x16x16f16(x.amin[tt], bmin, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < DPT; j++) {
+                    const float sv = HILO ? acc[tt][2 * j] + acc[tt][2 * j + 1] : acc[tt][j];
+                    const float sm = HILO ? accm[2 * j] + accm[2 * j + 1] : accm[j];
+                    tot[ti][tt][j] = fmaf(x.pe[tt][j], fmaf(d, sv, -(32.0f * dmin) * sm), tot[ti][tt][j]);
+                }
+            }
+        } else {
+            const float d = h2f(raw.d);
+            const uint32_t sel = 0x04000400u + 0x00010001u * (kg >> 1);   // byte kg / 16 of a scale pair
+#pragma unroll
+            for (int s = 0; s < 8; s++) {
+                // {sc, sc} exactly: byte sc + 128 under the exponent of 1024, minus 1152
+                const f16x2s sc2 = sk_bits(__builtin_amdgcn_perm(0x64646464u, raw.sc[s >> 1] ^ 0x80808080u, sel + 0x00020002u * (s & 1))) -
+                                   f16x2s{(_Float16)1152.0f, (_Float16)1152.0f};
+                uint32_t v0, v1, h0[2], h1[2], l0[2], l1[2];
+                Q::quants(raw, s, v0, v1);
+                sk_scale4_q6(v0, sc2, h0, l0);
+                sk_scale4_q6(v1, sc2, h1, l1);
+                const f16x8s bh = __builtin_bit_cast(f16x8s, u32x4{h0[0], h0[1], h1[0], h1[1]});
+                const f16x8s bl = __builtin_bit_cast(f16x8s, u32x4{l0[0], l0[1], l1[0], l1[1]});
+#pragma unroll
+                for (int tt = 0; tt < TOK; tt++) {
+                    acc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.av[tt][s], bh, acc[tt], 0, 0, 0);
+                    if constexpr (HILO) acc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.av[tt][s], bl, acc[tt], 0, 0, 0);
+                }
+                if constexpr (TOK > 1) __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int tt = 0; tt < TOK; tt++)
+#pragma unroll
+                for (int j = 0; j < DPT; j++) {
+                    const float sv = HILO ? acc[tt][2 * j] + acc[tt][2 * j + 1] : acc[tt][j];
+                    tot[ti][tt][j] = fmaf(x.pe[tt][j], d * sv, tot[ti][tt][j]);
+                }
+        }
+    };
+    auto column = [&](const A &x, A &next, uint32_t ci) {
+        if constexpr (DB) {
+            load_a(next, ci + 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        unit(x, ci, std::integral_constant<int, 0>{});
+        if constexpr (T > 1) unit(x, ci, std::integral_constant<int, 1>{});
+        if constexpr (T > 2) {
+            unit(x, ci, std::integral_constant<int, 2>{});
+            unit(x, ci, std::integral_constant<int, 3>{});
+        }
+    };
+
+    for (; tb0 < ntiles; tb0 += T * GR) {
+        // the first columns' A operands, then the first units: loads return in
+        // order, so unit 0 waits for the A operands and its own weights only
+        A x0, x1;
+        load_a(x0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) dma(u / T, tb0 + (u % T) * GR, u);
+#pragma unroll
+        for (int ti = 0; ti < T; ti++)
+#pragma unroll
+            for (int tt = 0; tt < TOK; tt++)
+#pragma unroll
+                for (int j = 0; j < DPT; j++) tot[ti][tt][j] = 0.0f;
+        buf = 0;
+        if constexpr (DB) {
+            for (uint32_t ci = 0; ci < Cw; ci += 2) {
+                column(x0, x1, ci);
+                if (ci + 1 < Cw) column(x1, x0, ci + 1);
+            }
+        } else {
+            column(x0, x1, 0);
+        }
+        // the wave's row sums over its ring (every DMA into it has landed, its
+        // reads are done)
+        wait_vm<0>();
+        float *pp = (float *)L + r16;
+#pragma unroll
+        for (int ti = 0; ti < T; ti++)
+#pragma unroll
+            for (int tt = 0; tt < TOK; tt++)
+#pragma unroll
+                for (int j = 0; j < DPT; j++)
+                    pp[(ti * MP + tt * TPT + (HILO ? 2 * kg + j : 4 * kg + j)) * 16] = tot[ti][tt][j];
         __syncthreads();
-        // the waves' partials in order
-        for (uint32_t i = t; i < MP * 16; i += 64 * W) {   // the launch's 64 W threads
-            const uint32_t m = i >> 4, c = i & 15, row = (tile0 + tl * GR) * 16 + c;
+        // the W waves' partials in wave order
+        for (uint32_t i = t; i < T * MP * 16; i += 64 * W) {
+            const uint32_t ti = i / (MP * 16), m = (i >> 4) % MP, c = i & 15, row = (tb0 + ti * GR) * 16 + c;
             if (m < M && row < N) {
-                // the W <= 16 waves' partials in wave order
-                float v = ordered_sum<16>(part + (size_t)buf * W * MP * 16 + i, W, MP * 16);
+                float v = ordered_sum<WMAX>(smem + i, W, NB * G::BUF / 4);
                 float *yp = a.y + (uint64_t)m * N + row;
                 if (a.residual) v = *yp + v;
                 *yp = v;
             }
         }
-        buf ^= 1u;
+        // the ring takes the next tiles' weights; nothing to wait for (the
+        // stores, too) after the last
+        if (tb0 + T * GR < ntiles) __syncthreads();
     }
 }
 
-static uint32_t sk_cus()
+template <class Q, bool HILO, int TOK, int T, int WMAX, bool DB>
+static hipError_t go_skinny_t(const GemvArgs &a, uint32_t waves, uint32_t ntiles, uint32_t grid, hipStream_t s)
 {
-    static uint32_t cus[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (!cus[dev]) {
-        int v = 0;
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;
-        cus[dev] = (uint32_t)v;
-    }
-    return cus[dev];
-}
-
-template <class Q, bool HILO, int TOK, int NB>
-static size_t sk_lds(uint32_t W)
-{
-    constexpr int MP = TOK * (HILO ? 8 : 16);
-    return (size_t)W * NB * SkGeom<Q>::BUF + 2ull * W * MP * 16 * 4;
-}
-
-template <class Q, bool HILO, int TOK, int NB>
-static hipError_t go_skinny_nb(const GemvArgs &a, hipStream_t s)
-{
-    const uint32_t W = a.K / 256, ntiles = (a.N + 15) / 16;
-    constexpr bool PRE = TOK > 1;
-    if (PRE)
-        hipLaunchKernelGGL(skinny_encode_kernel<HILO>, dim3(W, TOK), dim3(64), 0, s, a.x, a.M, a.K, a.ws, (uint32_t)TOK);
-    // up to one workgroup per CU, the tiles spread evenly over them
-    const uint32_t per = (ntiles + sk_cus() - 1) / sk_cus();
-    const uint32_t grid = (ntiles + per - 1) / per;
-    const size_t lds = sk_lds<Q, HILO, TOK, NB>(W);
-    hipLaunchKernelGGL((skinny_kernel<Q, HILO, TOK, NB, PRE>), dim3(grid), dim3(64 * W), lds, s, a, ntiles);
+    const size_t lds = (size_t)waves * sk_ring<Q, WMAX>() * SkGeom<Q>::BUF;
+    hipLaunchKernelGGL((skinny_kernel<Q, HILO, TOK, T, WMAX, DB>), dim3(grid), dim3(64 * waves), lds, s, a, ntiles);
     return hipGetLastError();
 }
 
-// the deepest tile ring that fits in LDS (160 KB)
-template <class Q, bool HILO, int TOK>
-static hipError_t go_skinny(const GemvArgs &a, hipStream_t s)
+// One workgroup per CU at most, the tiles spread evenly over them, T of them
+// at a time (one per workgroup: 1, two: 2, more: 4, where two columns' operands
+// of two A tiles leave the registers for it, else 2).  C columns a wave, the
+// fewest that need no more than WMAX waves.
+template <class Q, bool HILO, int TOK, int WMAX, bool DB>
+static hipError_t go_skinny_w(const GemvArgs &a, hipStream_t s)
 {
-    const uint32_t W = a.K / 256;
-    constexpr size_t LDS_MAX = 160 * 1024;
-    if (sk_lds<Q, HILO, TOK, 4>(W) <= LDS_MAX) return go_skinny_nb<Q, HILO, TOK, 4>(a, s);
-    if (sk_lds<Q, HILO, TOK, 3>(W) <= LDS_MAX) return go_skinny_nb<Q, HILO, TOK, 3>(a, s);
-    if (sk_lds<Q, HILO, TOK, 2>(W) <= LDS_MAX) return go_skinny_nb<Q, HILO, TOK, 2>(a, s);
-    return hipErrorNotSupported;
+    const uint32_t B = a.K / 256, ntiles = (a.N + 15) / 16;
+    const uint32_t C = (B + WMAX - 1) / WMAX, waves = (B + C - 1) / C;
+    const uint32_t cus = device_cu_count(), per = (ntiles + cus - 1) / cus, grid = (ntiles + per - 1) / per;
+    hipLaunchKernelGGL(skinny_encode_kernel<HILO>, dim3(B, TOK), dim3(256), 0, s, a.x, a.M, a.K, (uint8_t *)a.ws, (uint32_t)TOK);
+    if (per == 1) return go_skinny_t<Q, HILO, TOK, 1, WMAX, DB>(a, waves, ntiles, grid, s);
+    if (per == 2 || (DB && TOK == 2)) return go_skinny_t<Q, HILO, TOK, 2, WMAX, DB>(a, waves, ntiles, grid, s);
+    return go_skinny_t<Q, HILO, TOK, DB && TOK == 2 ? 2 : 4, WMAX, DB>(a, waves, ntiles, grid, s);
 }
 
 bool skinny_supported(const GemvArgs &a)
 {
-    if (a.type != T_Q4_K && a.type != T_Q5_K) return false;
-    if (a.M < 2 || a.M > 32 || a.K % 256 || a.K == 0) return false;
-    // waves per workgroup: up to 16 with one A tile (M <= 8), up to 12 with
-    // two, whose A operands need more registers
-    if (a.K > (a.M <= 8 ? 4096u : 3072u)) return false;
+    if (a.type != T_Q4_K && a.type != T_Q5_K && a.type != T_Q6_K) return false;
+    if (a.M < 1 || a.M > 32 || a.K % 256 || a.K == 0) return false;   // 1: the last of a longer run of rows
+    if (a.K > (1u << 16)) return false;   // 32-bit workspace offsets, with room
     if (!a.ws || a.ws_bytes < sk_ws_bytes(2, a.K / 256)) return false;
     return a.w_bytes + RRR_READ_SLACK < SK_OOB;
+}
+
+// Waves a workgroup: up to 12 (168 registers a lane; 16 waves would leave 128,
+// and two columns' operands of one A tile spill), 8 where two columns' operands
+// of two A tiles are held.
+template <class Q, bool HILO, int TOK>
+static hipError_t go_skinny(const GemvArgs &a, hipStream_t s)
+{
+    if (a.K <= 12 * 256) return go_skinny_w<Q, HILO, TOK, 12, false>(a, s);
+    return go_skinny_w<Q, HILO, TOK, TOK == 1 ? 12 : 8, true>(a, s);
 }
 
 template <class Q>
@@ -445,7 +605,11 @@ static hipError_t go_skinny_m(const GemvArgs &a, hipStream_t s)
 hipError_t launch_skinny(const GemvArgs &a, hipStream_t s)
 {
     if (!skinny_supported(a)) return hipErrorNotSupported;
-    return a.type == T_Q4_K ? go_skinny_m<SkQ4K>(a, s) : go_skinny_m<SkQ5K>(a, s);
+    switch (a.type) {
+    case T_Q4_K: return go_skinny_m<SkQ4K>(a, s);
+    case T_Q5_K: return go_skinny_m<SkQ5K>(a, s);
+    default: return go_skinny_m<SkQ6K>(a, s);
+    }
 }
 
 }  // namespace rrr
