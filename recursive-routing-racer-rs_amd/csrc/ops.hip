@@ -6,74 +6,102 @@
 namespace rrr {
 
 // ---------------------------------------------------------------------------
-// Standalone dequant to f32: bit-exact with phi4.rs:444-542.  One thread per
-// 16 consecutive output elements.  Every product below is exact in f32
-// (11-bit d times a 6-bit scale times a 6-bit quant), so each output carries
-// at most the single rounding of `q*s - m` that the Rust code performs.
-template <uint32_t TYPE>
-__global__ __launch_bounds__(256) void dequant_kernel(const uint8_t *__restrict__ W, uint64_t w_bytes,
-                                                       float *__restrict__ out, uint64_t n_groups)
+// Standalone dequant to f32: bit-exact with phi4.rs:444-542.  Every product
+// below is exact in f32 (11-bit d times a 6-bit scale times a 6-bit quant), so
+// each output carries at most the single rounding of `q*s - m` that the Rust
+// code performs.
+// Bound: HBM, nearly all of it the f32 stores.  A wave takes DQ_BLOCKS blocks,
+// every load of them issued first; lane l holds elements 4l .. 4l+3 of each,
+// so a store instruction writes one block's 1 KB as whole cache lines,
+// non-temporally (nothing here reads them again).  Q4_K 16384x3072 (230 MB):
+// 72 -> 33 us, 6.9 TB/s (Q6_K the same shape 79 -> 39 us); the form before gave
+// a thread 16 consecutive outputs, its four stores 64 bytes apart across the
+// lanes.
+constexpr int DQ_BLOCKS = 4;
+
+template <typename T>
+__device__ __forceinline__ T load_any(const uint8_t *p)   // any byte alignment
 {
-    const uint64_t gid = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (gid >= n_groups) return;
-    const uint64_t blk = gid >> 4;
-    const uint32_t e0 = (uint32_t)(gid & 15) * 16;
-    float v[16];
-    if constexpr (TYPE == T_Q4_K || TYPE == T_Q5_K) {
-        const uint32_t BS = TYPE == T_Q4_K ? 144 : 176;
-        const uint8_t *b = W + blk * BS;
-        const float d = h2f(b[0] | (b[1] << 8)), dmin = h2f(b[2] | (b[3] << 8));
-        const uint32_t sub = e0 / 32, j0 = e0 % 32, pair = sub / 2;
-        uint32_t sc, mn;
-        const uint8_t *q = b + 4;
-        if (sub < 4) {
-            sc = q[sub] & 63u;
-            mn = q[sub + 4] & 63u;
+    T v;
+    __builtin_memcpy(&v, p, sizeof(T));
+    return v;
+}
+
+// What lane l needs of a block, and its four elements.
+template <uint32_t TYPE>
+struct DqLane {
+    u32x4 hdr;
+    uint32_t q, h, x;
+    __device__ void load(const uint8_t *b, uint32_t lane)
+    {
+        const uint32_t j = 4 * (lane & 7);
+        if constexpr (TYPE == T_Q6_K) {
+            const uint32_t g = lane >> 5, quad = (lane >> 3) & 3;
+            q = load_any<uint32_t>(b + g * 64 + j + (quad & 1) * 32);
+            h = load_any<uint32_t>(b + 128 + g * 32 + j);
+            x = b[192 + g * 8 + (j >> 4) + 2 * quad];
+            hdr.x = load_any<uint16_t>(b + 208);
         } else {
-            const uint32_t i = sub - 4;
-            sc = (q[8 + i] & 0x0Fu) | ((uint32_t)(q[i] >> 6) << 4);
-            mn = (q[8 + i] >> 4) | ((uint32_t)(q[4 + i] >> 6) << 4);
+            hdr = load_any<u32x4>(b);
+            q = load_any<uint32_t>(b + (TYPE == T_Q4_K ? 16 : 48) + (lane >> 4) * 32 + j);
+            if constexpr (TYPE == T_Q5_K) h = load_any<uint32_t>(b + 16 + j);
         }
-        const float s = __fmul_rn(d, (float)sc), m = __fmul_rn(dmin, (float)mn);
-        const uint8_t *qs = b + (TYPE == T_Q4_K ? 16 : 48);
-        for (int i = 0; i < 16; i++) {
-            const uint32_t j = j0 + i;
-            const uint8_t qb = qs[pair * 32 + j];
-            uint32_t qi = (sub & 1) ? (qb >> 4) : (qb & 0xFu);
-            if constexpr (TYPE == T_Q5_K) qi |= ((uint32_t)(b[16 + j] >> sub) & 1u) << 4;
-            v[i] = __fsub_rn(__fmul_rn((float)qi, s), m);
-        }
-    } else if constexpr (TYPE == T_Q6_K) {
-        const uint8_t *b = W + blk * 210;
-        const float d = h2f(b[208] | (b[209] << 8));
-        const uint32_t g = e0 / 128, quad = (e0 % 128) / 32, l0 = e0 % 32;
-        const uint32_t is = g * 8 + l0 / 16 + 2 * quad;
-        const float ds = __fmul_rn(d, (float)(int8_t)b[192 + is]);
-        for (int i = 0; i < 16; i++) {
-            const uint32_t l = l0 + i;
-            const uint8_t qlb = b[g * 64 + l + (quad & 1) * 32];
-            const uint32_t lo = (quad < 2) ? (qlb & 0xFu) : (qlb >> 4);
-            const uint32_t hi = (b[128 + g * 32 + l] >> (2 * quad)) & 3u;
-            v[i] = __fmul_rn(ds, (float)((int)(lo | (hi << 4)) - 32));
-        }
-    } else {
-        const float *f = (const float *)W + gid * 16;
-        for (int i = 0; i < 16; i++) v[i] = f[i];
     }
-    float4 *o = (float4 *)(out + gid * 16);
-    for (int i = 0; i < 4; i++) o[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+    __device__ f32x4 values(uint32_t lane) const
+    {
+        f32x4 v;
+        const float d = h2f(hdr.x);
+        if constexpr (TYPE == T_Q6_K) {
+            const uint32_t quad = (lane >> 3) & 3;
+            const float ds = __fmul_rn(d, (float)(int8_t)x);
+            const uint32_t qi = ((q >> (quad & 2 ? 4 : 0)) & 0x0F0F0F0Fu) | (((h >> (2 * quad)) & 0x03030303u) << 4);
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = __fmul_rn(ds, (float)((int)byte_of(qi, i) - 32));
+        } else {
+            const uint32_t sub = lane >> 3;
+            uint32_t sc, mn;
+            scale_min_k4(sub, hdr.y, hdr.z, hdr.w, sc, mn);
+            const float s = __fmul_rn(d, (float)sc), m = __fmul_rn(h2f(hdr.x >> 16), (float)mn);
+            uint32_t qi = (q >> (4 * (sub & 1))) & 0x0F0F0F0Fu;
+            if constexpr (TYPE == T_Q5_K) qi |= ((h >> sub) & 0x01010101u) << 4;
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = __fsub_rn(__fmul_rn((float)byte_of(qi, i), s), m);
+        }
+        return v;
+    }
+};
+template <>
+struct DqLane<T_F32> {
+    f32x4 v;
+    __device__ void load(const uint8_t *b, uint32_t lane) { v = load_any<f32x4>(b + 16 * lane); }
+    __device__ f32x4 values(uint32_t) const { return v; }
+};
+
+// n_blocks blocks of 256 elements (BS bytes each)
+template <uint32_t TYPE, uint32_t BS>
+__global__ __launch_bounds__(256) void dequant_kernel(const uint8_t *__restrict__ W, float *__restrict__ out,
+                                                      uint64_t n_blocks)
+{
+    const uint32_t lane = threadIdx.x & 63;
+    const uint64_t b0 = ((uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * DQ_BLOCKS;
+    DqLane<TYPE> r[DQ_BLOCKS];
+#pragma unroll
+    for (int i = 0; i < DQ_BLOCKS; i++) r[i].load(W + min(b0 + i, n_blocks - 1) * BS, lane);
+#pragma unroll
+    for (int i = 0; i < DQ_BLOCKS; i++)
+        if (b0 + i < n_blocks) __builtin_nontemporal_store(r[i].values(lane), (f32x4 *)(out + (b0 + i) * 256) + lane);
 }
 
 hipError_t launch_dequant(uint32_t type, const uint8_t *W, uint64_t w_bytes, float *out, uint64_t n,
                           hipStream_t s)
 {
-    const uint64_t ng = n / 16;
-    const dim3 grid((unsigned)((ng + 255) / 256));
+    const uint64_t nb = n / 256;
+    const dim3 grid((unsigned)((nb + 4 * DQ_BLOCKS - 1) / (4 * DQ_BLOCKS)));
     switch (type) {
-    case T_Q4_K: hipLaunchKernelGGL(dequant_kernel<T_Q4_K>, grid, dim3(256), 0, s, W, w_bytes, out, ng); break;
-    case T_Q5_K: hipLaunchKernelGGL(dequant_kernel<T_Q5_K>, grid, dim3(256), 0, s, W, w_bytes, out, ng); break;
-    case T_Q6_K: hipLaunchKernelGGL(dequant_kernel<T_Q6_K>, grid, dim3(256), 0, s, W, w_bytes, out, ng); break;
-    case T_F32: hipLaunchKernelGGL(dequant_kernel<T_F32>, grid, dim3(256), 0, s, W, w_bytes, out, ng); break;
+    case T_Q4_K: hipLaunchKernelGGL((dequant_kernel<T_Q4_K, 144>), grid, dim3(256), 0, s, W, out, nb); break;
+    case T_Q5_K: hipLaunchKernelGGL((dequant_kernel<T_Q5_K, 176>), grid, dim3(256), 0, s, W, out, nb); break;
+    case T_Q6_K: hipLaunchKernelGGL((dequant_kernel<T_Q6_K, 210>), grid, dim3(256), 0, s, W, out, nb); break;
+    case T_F32: hipLaunchKernelGGL((dequant_kernel<T_F32, 1024>), grid, dim3(256), 0, s, W, out, nb); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
