@@ -86,6 +86,7 @@ struct rrr_ctx {
     void *att_scratch;  // attention: per-KV-head counters (zero between calls) and split partials
     void *gemm_ws;      // GEMM_WS_BYTES: prefill GEMM partials of split K; the skinny GEMV's encoded
                         // activations; the split-K logits' partials (stream order keeps the users apart)
+    void *gemm_wx;      // GEMM_WX_BYTES: weights expanded to f16 for the long-prompt GEMM
     void *logits_cnt;   // split-K logits: per-slab counters (zero between calls)
     std::unordered_set<rrr_buf *> bufs;
     std::unordered_set<rrr_graph *> graphs;
@@ -194,7 +195,7 @@ int rrr_init(int device, rrr_ctx **out)
     ctx->async = ctx->capturing = ctx->timer_started = false;
     ctx->stream = nullptr;
     ctx->ev0 = ctx->ev1 = nullptr;
-    ctx->scratch = ctx->att_scratch = ctx->gemm_ws = ctx->logits_cnt = nullptr;
+    ctx->scratch = ctx->att_scratch = ctx->gemm_ws = ctx->gemm_wx = ctx->logits_cnt = nullptr;
     if (!ctx->nodevice) {
         int n = rrr_device_count();
         if (device >= n) {
@@ -209,6 +210,7 @@ int rrr_init(int device, rrr_ctx **out)
         if (e == hipSuccess) e = hipMalloc(&ctx->att_scratch, attention_scratch_bytes());
         if (e == hipSuccess) e = hipMemset(ctx->att_scratch, 0, attention_scratch_bytes());
         if (e == hipSuccess) e = hipMalloc(&ctx->gemm_ws, GEMM_WS_BYTES);
+        if (e == hipSuccess) e = hipMalloc(&ctx->gemm_wx, GEMM_WX_BYTES);
         if (e == hipSuccess) e = hipMalloc(&ctx->logits_cnt, logits_counter_bytes());
         if (e == hipSuccess) e = hipMemset(ctx->logits_cnt, 0, logits_counter_bytes());
         if (e == hipSuccess) e = hipDeviceSynchronize();
@@ -216,6 +218,7 @@ int rrr_init(int device, rrr_ctx **out)
         if (e == hipSuccess && attention_static_setup(device, &static_scratch) != RRR_OK) e = hipErrorInvalidSymbol;
         if (e != hipSuccess) {
             if (ctx->logits_cnt) (void)hipFree(ctx->logits_cnt);
+            if (ctx->gemm_wx) (void)hipFree(ctx->gemm_wx);
             if (ctx->gemm_ws) (void)hipFree(ctx->gemm_ws);
             if (ctx->att_scratch) (void)hipFree(ctx->att_scratch);
             if (ctx->scratch) (void)hipFree(ctx->scratch);
@@ -256,6 +259,7 @@ int rrr_destroy(rrr_ctx *ctx)
         (void)hipFree(ctx->scratch);
         (void)hipFree(ctx->att_scratch);
         (void)hipFree(ctx->gemm_ws);
+        (void)hipFree(ctx->gemm_wx);
         (void)hipFree(ctx->logits_cnt);
         (void)hipEventDestroy(ctx->ev0);
         (void)hipEventDestroy(ctx->ev1);
@@ -486,6 +490,7 @@ static int gemv_prepare(rrr_ctx *ctx, const rrr_buf *X, uint64_t x_floats, const
     a.residual = residual;
     a.ws = ctx->gemm_ws;
     a.ws_bytes = GEMM_WS_BYTES;
+    a.wx = ctx->gemm_wx;
     return RRR_OK;
 }
 
@@ -587,7 +592,7 @@ int rrr_gemm_bf16(rrr_ctx *ctx, const rrr_buf *X, const rrr_buf *W, uint32_t typ
         return fail(RRR_ERR_INVALID_ARG, "%s: X and Y must be 16-byte aligned", what);
     TRY(device_ready(ctx));
     hipError_t e = launch_gemm_bf16((const uint16_t *)X->ptr, (const uint8_t *)W->ptr, type, (float *)Y->ptr, K, N, M,
-                                    (float *)ctx->gemm_ws, GEMM_WS_BYTES, ctx->stream);
+                                    (float *)ctx->gemm_ws, GEMM_WS_BYTES, ctx->gemm_wx, ctx->stream);
     if (e == hipErrorNotSupported) return fail(RRR_ERR_UNSUPPORTED, "%s: shape not supported by the kernels", what);
     return finish(ctx, e, what);
 }
@@ -942,7 +947,7 @@ int rrr_gemm_f16(rrr_ctx *ctx, const rrr_buf *X, const rrr_buf *row_scale, const
     TRY(device_ready(ctx));
     return finish(ctx, launch_gemm_f16((const uint16_t *)X->ptr, row_scale ? (const float *)row_scale->ptr : nullptr,
                                        (const uint8_t *)W->ptr, type, (float *)Y->ptr, K, N, M, accumulate != 0,
-                                       (float *)ctx->gemm_ws, GEMM_WS_BYTES, ctx->stream),
+                                       (float *)ctx->gemm_ws, GEMM_WS_BYTES, ctx->gemm_wx, ctx->stream),
                   what);
 }
 
@@ -978,7 +983,7 @@ int rrr_gemm_f16_rmsnorm(rrr_ctx *ctx, const rrr_buf *X, const rrr_buf *row_scal
                   launch_gemm_f16_rmsnorm((const uint16_t *)X->ptr, row_scale ? (const float *)row_scale->ptr : nullptr,
                                           (const uint8_t *)W->ptr, type, (float *)Y->ptr, K, N, M, accumulate != 0,
                                           (const float *)gamma->ptr, eps, (uint16_t *)y16->ptr, (float *)ctx->gemm_ws,
-                                          GEMM_WS_BYTES, ctx->stream),
+                                          GEMM_WS_BYTES, ctx->gemm_wx, ctx->stream),
                   what);
 }
 
@@ -1010,7 +1015,7 @@ int rrr_gemm_f16_rope_kv_rows(rrr_ctx *ctx, const rrr_buf *X, const rrr_buf *W, 
     return finish(ctx,
                   launch_gemm_f16_rope_kv((const uint16_t *)X->ptr, (const uint8_t *)W->ptr, type, (float *)qkv->ptr, K,
                                           N, M, r, rows, (uint16_t *)k_cache->ptr, (uint16_t *)v_cache->ptr,
-                                          (float *)ctx->gemm_ws, GEMM_WS_BYTES, ctx->stream),
+                                          (float *)ctx->gemm_ws, GEMM_WS_BYTES, ctx->gemm_wx, ctx->stream),
                   what);
 }
 

@@ -601,6 +601,15 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce(const float *__restric
     *y = v;
 }
 
+// What follows the GEMM where no split reduction takes it in: the rope_kv_store
+// or the RMSNorm of Y's rows.
+static hipError_t gemm_then(float *Y, uint32_t N, uint32_t M, const GemmNorm *nrm, const GemmRope *rp, hipStream_t s)
+{
+    if (rp) return launch_rope_kv_store(Y, rp->r, rp->kc, rp->vc, s, rp->rows);
+    if (nrm) return launch_rmsnorm_f16(Y, nrm->gamma, nrm->out, M, N, nrm->eps, s);
+    return hipSuccess;
+}
+
 template <template <int> class QT, int BM, int BN, int BK, bool ACC>
 static hipError_t go_gemm(const uint16_t *X, const float *rscale, const uint8_t *W, float *Y, uint32_t K, uint32_t N,
                           uint32_t M, uint32_t mrows, uint32_t S, float *ws, const GemmNorm *nrm, const GemmRope *rp,
@@ -608,8 +617,6 @@ static hipError_t go_gemm(const uint16_t *X, const float *rscale, const uint8_t 
 {
     constexpr size_t lds = gemm_lds_bytes<BM, BN, BK>;
     static_assert(lds <= 160 * 1024, "LDS per workgroup");
-    // the fused reductions take every one of the M rows
-    if ((nrm || rp) && mrows != M) return hipErrorInvalidValue;
     const uint32_t tiles_n = N / BN, tiles = tiles_n * (M / BM);
     if (S > 1)
         hipLaunchKernelGGL((gemm_dq_kernel<QT, BM, BN, BK, ACC, true>), dim3(tiles * S), dim3(512), lds, s, X, W, Y, K,
@@ -617,23 +624,11 @@ static hipError_t go_gemm(const uint16_t *X, const float *rscale, const uint8_t 
     else
         hipLaunchKernelGGL((gemm_dq_kernel<QT, BM, BN, BK, ACC, false>), dim3(tiles), dim3(512), lds, s, X, W, Y, K,
                            N, M, tiles_n, rscale, 1u, nullptr, mrows);
-    if (S > 1 && rp) {
-        // the reduction is the rope_kv_store's first step
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        return launch_splitk_rope_kv_store(ws, S, M, Y, rp->r, rp->rows, rp->kc, rp->vc, s);
-    }
-    if (rp) {
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        return launch_rope_kv_store(Y, rp->r, rp->kc, rp->vc, s, rp->rows);
-    }
-    if (S > 1 && nrm) {
-        // the reduction also writes the rows' RMSNorm
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        return launch_splitk_reduce_rmsnorm(ws, S, M, N, Y, rscale, ACC, nrm->gamma, nrm->eps, nrm->out, s);
-    }
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    // the reduction is the rope_kv_store's first step, or also writes the rows' RMSNorm
+    if (S > 1 && rp) return launch_splitk_rope_kv_store(ws, S, M, Y, rp->r, rp->rows, rp->kc, rp->vc, s);
+    if (S > 1 && nrm) return launch_splitk_reduce_rmsnorm(ws, S, M, N, Y, rscale, ACC, nrm->gamma, nrm->eps, nrm->out, s);
     if (S > 1) {
         const uint64_t quads = (uint64_t)mrows * N / 4;
         const dim3 grid((unsigned)((quads + 255) / 256));
@@ -648,12 +643,8 @@ static hipError_t go_gemm(const uint16_t *X, const float *rscale, const uint8_t 
         }
 #undef RRR_SKR_CASE
     }
-    if (nrm) {
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        return launch_rmsnorm_f16(Y, nrm->gamma, nrm->out, M, N, nrm->eps, s);
-    }
-    return hipGetLastError();
+    e = hipGetLastError();
+    return e == hipSuccess ? gemm_then(Y, N, M, nrm, rp, s) : e;
 }
 
 // Splits of K for a grid of `tiles` tiles: at most as many as keep every
@@ -676,22 +667,40 @@ static uint32_t gemm_splits(uint32_t tiles, uint32_t K, uint32_t M, uint32_t N, 
     return best;
 }
 
+// How gemm_dq_kernel takes a shape: 256 x 128 tiles when they cover at least
+// half of the CUs, or with K split to do so; else 128 x 64 (with K steps of 128
+// so each barrier covers as much MFMA work), K split the same way when those
+// tiles are few.  us: its time, measured over 128 to 2,048 rows of nine shapes:
+// a round of 256 x 128 tiles 0.80 to 1.05 us per 64 k (few CUs busy to all) and
+// 6 us of stores and start-up, one of 128 x 64 tiles 0.65 to 0.85 us per 128 k
+// and 3 us, a split reduction 8 us.
+struct GemmPlan {
+    bool big;
+    uint32_t S;
+    float us;
+};
+static GemmPlan gemm_plan(uint32_t K, uint32_t N, uint32_t M, bool split, size_t ws_bytes)
+{
+    const uint32_t B = K / 256;
+    if (M % 256 == 0 && N % 128 == 0) {
+        const uint32_t tiles = (N / 128) * (M / 256), S = split ? gemm_splits(tiles, K, M, N, ws_bytes) : 1u;
+        const float k = (float)((B + S - 1) / S);
+        if (tiles * S >= 128)
+            return {true, S, gemm_rounds(tiles * S, k * 4 * 0.80f, k * 4 * 0.25f, 6.0f) + (S > 1 ? 8.0f : 0.0f)};
+    }
+    const uint32_t tiles = (N / 64) * (M / 128), S = split ? gemm_splits(tiles, K, M, N, ws_bytes) : 1u;
+    const float k = (float)((B + S - 1) / S);
+    return {false, S, gemm_rounds(tiles * S, k * 2 * 0.65f, k * 2 * 0.20f, 3.0f) + (S > 1 ? 8.0f : 0.0f)};
+}
+
 template <template <int> class QT, bool ACC>
 static hipError_t go_gemm_t(const uint16_t *X, const float *rscale, const uint8_t *W, float *Y, uint32_t K,
                             uint32_t N, uint32_t M, uint32_t mrows, float *ws, size_t ws_bytes, const GemmNorm *nrm,
                             const GemmRope *rp, hipStream_t s)
 {
-    // 256 x 128 tiles when they cover at least half of the CUs, or with K
-    // split to do so; else 128 x 64 (with K steps of 128 so each barrier
-    // covers as much MFMA work), K split the same way when those tiles are few
-    if (M % 256 == 0 && N % 128 == 0) {
-        const uint32_t tiles = (N / 128) * (M / 256);
-        const uint32_t S = ws ? gemm_splits(tiles, K, M, N, ws_bytes) : 1u;
-        if (tiles * S >= 128)
-            return go_gemm<QT, 256, 128, 64, ACC>(X, rscale, W, Y, K, N, M, mrows, S, ws, nrm, rp, s);
-    }
-    const uint32_t S = ws ? gemm_splits((N / 64) * (M / 128), K, M, N, ws_bytes) : 1u;
-    return go_gemm<QT, 128, 64, 128, ACC>(X, rscale, W, Y, K, N, M, mrows, S, ws, nrm, rp, s);
+    const GemmPlan p = gemm_plan(K, N, M, ws != nullptr, ws_bytes);
+    if (p.big) return go_gemm<QT, 256, 128, 64, ACC>(X, rscale, W, Y, K, N, M, mrows, p.S, ws, nrm, rp, s);
+    return go_gemm<QT, 128, 64, 128, ACC>(X, rscale, W, Y, K, N, M, mrows, p.S, ws, nrm, rp, s);
 }
 
 bool gemm_supported(uint32_t type, uint32_t K, uint32_t N, uint32_t M, uint64_t x_bytes)
@@ -702,10 +711,18 @@ bool gemm_supported(uint32_t type, uint32_t K, uint32_t N, uint32_t M, uint64_t 
 
 template <bool ACC>
 static hipError_t go_gemm_q(const uint16_t *X, const float *rscale, const uint8_t *W, uint32_t type, float *Y,
-                            uint32_t K, uint32_t N, uint32_t M, uint32_t mrows, float *ws, size_t ws_bytes,
+                            uint32_t K, uint32_t N, uint32_t M, uint32_t mrows, float *ws, size_t ws_bytes, void *wx,
                             hipStream_t s, const GemmNorm *nrm = nullptr, const GemmRope *rp = nullptr)
 {
     if (!gemm_supported(type, K, N, M, (uint64_t)M * K * 2) || mrows == 0 || mrows > M) return hipErrorNotSupported;
+    // the fused reductions and what follows take every one of the M rows
+    if ((nrm || rp) && mrows != M) return hipErrorInvalidValue;
+    // the weights expanded to f16 first where that is faster: long prompts,
+    // and row counts that leave the 256 x 128 tiles' rounds part empty
+    if (wx && gemm_wide_cost(K, N, mrows, GEMM_WX_BYTES) < 0.97f * gemm_plan(K, N, M, ws != nullptr, ws_bytes).us) {
+        const hipError_t e = launch_gemm_wide(X, rscale, W, type, Y, K, N, M, mrows, ACC, wx, GEMM_WX_BYTES, s);
+        return e == hipSuccess ? gemm_then(Y, N, M, nrm, rp, s) : e;
+    }
     switch (type) {
     case T_Q4_K: return go_gemm_t<GqQ4K, ACC>(X, rscale, W, Y, K, N, M, mrows, ws, ws_bytes, nrm, rp, s);
     case T_Q5_K: return go_gemm_t<GqQ5K, ACC>(X, rscale, W, Y, K, N, M, mrows, ws, ws_bytes, nrm, rp, s);
@@ -791,7 +808,7 @@ static uint32_t gemm_chunk_rows(uint32_t M, uint32_t K, size_t ws_bytes)
 
 // X (bf16 or f32, M x K) . W^T in row chunks through the f16 GEMM.
 static hipError_t gemm_rows(const void *X, bool f32, const uint8_t *W, uint32_t type, float *Y, uint32_t K,
-                            uint32_t N, uint32_t M, void *ws, size_t ws_bytes, hipStream_t s)
+                            uint32_t N, uint32_t M, void *ws, size_t ws_bytes, void *wx, hipStream_t s)
 {
     const uint32_t mc = ws ? gemm_chunk_rows(M, K, ws_bytes) : 0u;
     if (!mc || !gemm_supported(type, K, N, mc, (uint64_t)mc * K * 2)) return hipErrorNotSupported;
@@ -814,16 +831,16 @@ static hipError_t gemm_rows(const void *X, bool f32, const uint8_t *W, uint32_t 
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         e = go_gemm_q<false>(Xh, f32 ? rscale : nullptr, W, type, Y + (uint64_t)m0 * N, K, N, mp, rows, part,
-                             part_bytes, s);
+                             part_bytes, wx, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
 }
 
 hipError_t launch_gemm_bf16(const uint16_t *X, const uint8_t *W, uint32_t type, float *Y, uint32_t K, uint32_t N,
-                            uint32_t M, float *ws, size_t ws_bytes, hipStream_t s)
+                            uint32_t M, float *ws, size_t ws_bytes, void *wx, hipStream_t s)
 {
-    return gemm_rows(X, false, W, type, Y, K, N, M, ws, ws_bytes, s);
+    return gemm_rows(X, false, W, type, Y, K, N, M, ws, ws_bytes, wx, s);
 }
 
 bool gemm_rows_supported(uint32_t type, uint32_t K, uint32_t N, uint32_t M, size_t ws_bytes)
@@ -833,27 +850,27 @@ bool gemm_rows_supported(uint32_t type, uint32_t K, uint32_t N, uint32_t M, size
 }
 
 hipError_t launch_gemm_f32_rows(const float *X, const uint8_t *W, uint32_t type, float *Y, uint32_t K, uint32_t N,
-                                uint32_t M, void *ws, size_t ws_bytes, hipStream_t s)
+                                uint32_t M, void *ws, size_t ws_bytes, void *wx, hipStream_t s)
 {
-    return gemm_rows(X, true, W, type, Y, K, N, M, ws, ws_bytes, s);
+    return gemm_rows(X, true, W, type, Y, K, N, M, ws, ws_bytes, wx, s);
 }
 
 hipError_t launch_gemm_f16(const uint16_t *X, const float *rscale, const uint8_t *W, uint32_t type, float *Y,
-                           uint32_t K, uint32_t N, uint32_t M, bool accumulate, float *ws, size_t ws_bytes,
+                           uint32_t K, uint32_t N, uint32_t M, bool accumulate, float *ws, size_t ws_bytes, void *wx,
                            hipStream_t s)
 {
-    return accumulate ? go_gemm_q<true>(X, rscale, W, type, Y, K, N, M, M, ws, ws_bytes, s)
-                      : go_gemm_q<false>(X, rscale, W, type, Y, K, N, M, M, ws, ws_bytes, s);
+    return accumulate ? go_gemm_q<true>(X, rscale, W, type, Y, K, N, M, M, ws, ws_bytes, wx, s)
+                      : go_gemm_q<false>(X, rscale, W, type, Y, K, N, M, M, ws, ws_bytes, wx, s);
 }
 
 hipError_t launch_gemm_f16_rmsnorm(const uint16_t *X, const float *rscale, const uint8_t *W, uint32_t type, float *Y,
                                    uint32_t K, uint32_t N, uint32_t M, bool accumulate, const float *gamma, float eps,
-                                   uint16_t *out16, float *ws, size_t ws_bytes, hipStream_t s)
+                                   uint16_t *out16, float *ws, size_t ws_bytes, void *wx, hipStream_t s)
 {
     if (!splitk_reduce_rmsnorm_supported(N)) return hipErrorNotSupported;
     const GemmNorm nrm{gamma, eps, out16};
-    return accumulate ? go_gemm_q<true>(X, rscale, W, type, Y, K, N, M, M, ws, ws_bytes, s, &nrm)
-                      : go_gemm_q<false>(X, rscale, W, type, Y, K, N, M, M, ws, ws_bytes, s, &nrm);
+    return accumulate ? go_gemm_q<true>(X, rscale, W, type, Y, K, N, M, M, ws, ws_bytes, wx, s, &nrm)
+                      : go_gemm_q<false>(X, rscale, W, type, Y, K, N, M, M, ws, ws_bytes, wx, s, &nrm);
 }
 
 // The gate/up GEMM with silu(gate) * up in its epilogue into ws (M x F
@@ -886,11 +903,11 @@ hipError_t launch_gemm_f16_silu_f16(const uint16_t *X, const uint8_t *W, uint32_
 
 hipError_t launch_gemm_f16_rope_kv(const uint16_t *X, const uint8_t *W, uint32_t type, float *Y, uint32_t K,
                                    uint32_t N, uint32_t M, const RopeArgs &r, uint32_t rows, uint16_t *kc,
-                                   uint16_t *vc, float *ws, size_t ws_bytes, hipStream_t s)
+                                   uint16_t *vc, float *ws, size_t ws_bytes, void *wx, hipStream_t s)
 {
     if (!splitk_rope_kv_store_supported(r) || r.row_stride != N || rows > M) return hipErrorNotSupported;
     const GemmRope rp{r, rows, kc, vc};
-    return go_gemm_q<false>(X, nullptr, W, type, Y, K, N, M, M, ws, ws_bytes, s, nullptr, &rp);
+    return go_gemm_q<false>(X, nullptr, W, type, Y, K, N, M, M, ws, ws_bytes, wx, s, nullptr, &rp);
 }
 
 }  // namespace rrr

@@ -612,7 +612,7 @@ static hipError_t launch_rows(const GemvArgs &a, hipStream_t s)
     if (gemv_mq_tokens_supported(a)) return launch_gemv_mq_tokens(a, s);
     const bool gemm = batched_gemm_route(a);
     if (skinny_supported(a) && (a.M <= 16 || gemm || (a.type != T_Q6_K && a.K <= 3072))) return launch_skinny(a, s);
-    if (gemm) return launch_gemm_f32_rows(a.x, a.W, a.type, a.y, a.K, a.N, a.M, a.ws, a.ws_bytes, s);
+    if (gemm) return launch_gemm_f32_rows(a.x, a.W, a.type, a.y, a.K, a.N, a.M, a.ws, a.ws_bytes, a.wx, s);
     GemvArgs r = a;
     r.M = a.M < 16 ? a.M : 16;
     if (!skinny_supported(r)) return hipErrorNotSupported;

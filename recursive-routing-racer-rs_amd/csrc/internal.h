@@ -37,6 +37,7 @@ struct GemvArgs {
     uint32_t residual;    // y += result instead of y = result
     void *ws;             // device workspace of the skinny path's encoded activations
     uint64_t ws_bytes;
+    void *wx;             // workspace of expanded weights (GEMM_WX_BYTES), for many rows
     uint32_t pair;        // W holds 2N rows [gate | up]; y[n] = silu(gate row n) * (up row n)
     // rope_kv_store in the epilogue (y = qkv of one token at rope.pos): RoPE
     // pairs rotated before they are stored, K and V also stored as f16 into
@@ -135,19 +136,36 @@ hipError_t launch_attention_prefill(const float *qkv, uint32_t row_stride, uint3
 // multiplied by rscale[m] (a power of two: exact) first.  ws (ws_bytes, may
 // be null) holds the fp32 partials when K is split.
 constexpr size_t GEMM_WS_BYTES = 48ull << 20;
+// wx: GEMM_WX_BYTES for weights expanded to f16 (gemm_wide.hip), taken in column
+// parts where they need more; null: the weights are never expanded.
+constexpr size_t GEMM_WX_BYTES = 128ull << 20;
 bool gemm_supported(uint32_t type, uint32_t K, uint32_t N, uint32_t M, uint64_t x_bytes);
 // bf16 X (any M >= 1, X and Y 16-byte aligned): converted to f16 in row
 // chunks inside ws, each chunk zero-padded to a multiple of 128 rows
 hipError_t launch_gemm_bf16(const uint16_t *X, const uint8_t *W, uint32_t type, float *Y, uint32_t K, uint32_t N,
-                            uint32_t M, float *ws, size_t ws_bytes, hipStream_t s);
+                            uint32_t M, float *ws, size_t ws_bytes, void *wx, hipStream_t s);
 // f32 X (the batched GEMV above 16 rows): each row chunk as f16 block floating
 // point (row m scaled by a power of two, undone exactly on Y's row) in ws
 bool gemm_rows_supported(uint32_t type, uint32_t K, uint32_t N, uint32_t M, size_t ws_bytes);
 hipError_t launch_gemm_f32_rows(const float *X, const uint8_t *W, uint32_t type, float *Y, uint32_t K, uint32_t N,
-                                uint32_t M, void *ws, size_t ws_bytes, hipStream_t s);
+                                uint32_t M, void *ws, size_t ws_bytes, void *wx, hipStream_t s);
 hipError_t launch_gemm_f16(const uint16_t *X, const float *rscale, const uint8_t *W, uint32_t type, float *Y,
-                           uint32_t K, uint32_t N, uint32_t M, bool accumulate, float *ws, size_t ws_bytes,
+                           uint32_t K, uint32_t N, uint32_t M, bool accumulate, float *ws, size_t ws_bytes, void *wx,
                            hipStream_t s);
+// us of `tiles` tiles in rounds of 256 (one a CU): each `base` + `load` times
+// the round's share of the CUs + `fixed`.
+inline float gemm_rounds(uint32_t tiles, float base, float load, float fixed)
+{
+    const uint32_t full = tiles / 256, rest = tiles % 256;
+    return full * (base + load + fixed) + (rest ? base + load * (rest / 256.0f) + fixed : 0.0f);
+}
+// The same product with W expanded to f16 first (gemm_wide.hip), whole K: the
+// bits of launch_gemm_f16 without split K.  mrows <= M: the rows stored.
+// gemm_wide_cost: its time in us, for the choice between the two.
+float gemm_wide_cost(uint32_t K, uint32_t N, uint32_t M, size_t wx_bytes);
+hipError_t launch_gemm_wide(const uint16_t *X, const float *rscale, const uint8_t *W, uint32_t type, float *Y,
+                            uint32_t K, uint32_t N, uint32_t M, uint32_t mrows, bool acc, void *wx, size_t wx_bytes,
+                            hipStream_t s);
 // the same GEMM, then the RMSNorm (gamma, eps) of Y's rows in f16 into out16:
 // with K split, inside the split reduction (splitk_reduce_rmsnorm_kernel),
 // else the rmsnorm launch after the GEMM; N % 4 == 0, N <= 8192
@@ -158,7 +176,7 @@ struct GemmNorm {
 };
 hipError_t launch_gemm_f16_rmsnorm(const uint16_t *X, const float *rscale, const uint8_t *W, uint32_t type, float *Y,
                                    uint32_t K, uint32_t N, uint32_t M, bool accumulate, const float *gamma, float eps,
-                                   uint16_t *out16, float *ws, size_t ws_bytes, hipStream_t s);
+                                   uint16_t *out16, float *ws, size_t ws_bytes, void *wx, hipStream_t s);
 // the QKV GEMM (accumulate 0, no row scale) of the prompt's M rows into the
 // qkv rows Y, then the rope_kv_store of its first `rows` rows at positions
 // r.pos ..: with K split, inside the split reduction
@@ -170,7 +188,7 @@ struct GemmRope {
 };
 hipError_t launch_gemm_f16_rope_kv(const uint16_t *X, const uint8_t *W, uint32_t type, float *Y, uint32_t K,
                                    uint32_t N, uint32_t M, const RopeArgs &r, uint32_t rows, uint16_t *kc,
-                                   uint16_t *vc, float *ws, size_t ws_bytes, hipStream_t s);
+                                   uint16_t *vc, float *ws, size_t ws_bytes, void *wx, hipStream_t s);
 // the gate/up GEMM (N = 2F: F gate rows, F up rows) with silu(gate) * up in
 // its epilogue into ws (M x F f32), then silu_gate_f16's block floating
 // point rows from those values (launch_f16_rows_scaled)
