@@ -592,13 +592,11 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
     }
 }
 
-// Causal prefill attention on the matrix cores.  Workgroup (g, tb): query
-// heads g*HPK .. g*HPK+HPK-1, of KV head g / hsplit (hsplit workgroups share
-// a KV group's heads_per_kv = hsplit * HPK heads; hsplit 1: all of them),
-// tokens tb*16 .. tb*16+15 (lane l's token is l % 16); its ATTM_WAVES
-// waves take every ATTM_WAVES-th block of 32 cache rows and merge their
-// (max, sum, output) at the end in a fixed order.  Per block and per query
-// head h of the group:
+// Causal prefill attention on the matrix cores, short prompts (attn_flash.hip
+// has the form for more).  Workgroup (g, tb): query head g, of KV head g /
+// heads_per_kv, tokens tb*16 .. tb*16+15 (lane l's token is l % 16); its
+// ATTM_WAVES waves take every ATTM_WAVES-th block of 32 cache rows and merge
+// their (max, sum, output) at the end in a fixed order.  Per block:
 //   S^T = K . Q^T    (v_mfma_f32_16x16x32_f16, keys x tokens, K from the f16
 //                     cache as A operands, Q^T as B operands in f16 hi + lo,
 //                     so the scores carry ~2^-22 of Q's rounding)
@@ -618,8 +616,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
 // [2^13, 2^14), inside f16's range whatever the activations' size) and of
 // P * 2^12 (P <= 8), undone exactly on the scores and at the end; the lo
 // parts then stay in f16's normal range, where they keep their precision.
-// The Q^T operands sit in LDS (one head's are read per block), so the
-// accumulators need no moves between register files.
+// The Q^T operands sit in LDS and are read per block.
 constexpr uint32_t ATTM_LD = 36;   // f16 per V^T row in LDS (32 keys + pad; 72-byte rows)
 constexpr float ATTM_PS = 4096.0f;
 constexpr uint32_t ATTM_WAVES = 4, ATTM_OLD = ATT_HD + 4;   // waves; floats per merged output row (padded)
@@ -631,41 +628,40 @@ __device__ __forceinline__ void wave_lds_order()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int HPK>
 struct AttmLds {
     static constexpr size_t VT = (size_t)ATTM_WAVES * ATT_HD * ATTM_LD * 2;            // V^T per wave
-    static constexpr size_t O = (size_t)ATTM_WAVES * HPK * 16 * ATTM_OLD * 4;          // merge: outputs
-    static constexpr size_t ML = (size_t)ATTM_WAVES * HPK * 16 * 2 * 4;                // merge: max, sum
-    static constexpr size_t Q = (size_t)HPK * 4 * 2 * 64 * 16;                        // Q^T operands, hi + lo
+    static constexpr size_t O = (size_t)ATTM_WAVES * 16 * ATTM_OLD * 4;          // merge: outputs
+    static constexpr size_t ML = (size_t)ATTM_WAVES * 16 * 2 * 4;                // merge: max, sum
+    static constexpr size_t Q = (size_t)4 * 2 * 64 * 16;                        // Q^T operands, hi + lo
     // the loop's V^T and Q^T share their bytes with the merge's outputs
-    static constexpr size_t CW = (size_t)HPK * 16 * (ATTM_WAVES + 1) * 4;             // merge: weights, scale
+    static constexpr size_t CW = (size_t)16 * (ATTM_WAVES + 1) * 4;             // merge: weights, scale
     static constexpr size_t LOOP = VT + Q, MAIN = LOOP > O ? LOOP : O;
     static constexpr size_t BYTES = MAIN + ML + CW;
 };
 
-template <int HPK, bool F16OUT>
+template <bool F16OUT>
 __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(const float *__restrict__ qkv, uint32_t row_stride,
                                                                const uint16_t *__restrict__ kc,
                                                                const uint16_t *__restrict__ vc,
                                                                void *__restrict__ out, uint32_t rows, uint32_t pos0,
-                                                               uint32_t kv_stride, float qscale, uint32_t hsplit)
+                                                               uint32_t kv_stride, float qscale, uint32_t heads_per_kv)
 {
     typedef _Float16 h8 __attribute__((ext_vector_type(8)));
     typedef _Float16 h4 __attribute__((ext_vector_type(4)));
     typedef float f4 __attribute__((ext_vector_type(4)));
-    using LD = AttmLds<HPK>;
+    using LD = AttmLds;
     __shared__ __attribute__((aligned(16))) uint8_t sm[LD::BYTES];
     const uint32_t wv = threadIdx.x >> 6;
     _Float16 *vt = (_Float16 *)sm + (size_t)wv * ATT_HD * ATTM_LD;   // this wave's V^T
     float *mo = (float *)sm;                                        // merge outputs (after the loop)
     float *mml = (float *)(sm + LD::MAIN);                          // merge max / sum
-    float *mcw = (float *)(sm + LD::MAIN + LD::ML);                 // merge weights and scale per (head, token)
+    float *mcw = (float *)(sm + LD::MAIN + LD::ML);                 // merge weights and scale per token
     h8 *qop = (h8 *)(sm + LD::VT);                                  // Q^T operands [h][kk][hi, lo][lane]
     const uint32_t g = blockIdx.x, tb = blockIdx.y, l = threadIdx.x & 63, n = l & 15, grp = l >> 4;
     const uint32_t tok = tb * 16 + n, tq = min(tok, rows - 1), tpos = pos0 + tq;
     const uint32_t last = pos0 + min(tb * 16 + 15, rows - 1);      // the last cache row the block's tokens see
     const uint32_t nblk = last / 32 + 1;
-    const uint16_t *kbase = kc + (size_t)(g / hsplit) * ATT_HD, *vbase = vc + (size_t)(g / hsplit) * ATT_HD;
+    const uint16_t *kbase = kc + (size_t)(g / heads_per_kv) * ATT_HD, *vbase = vc + (size_t)(g / heads_per_kv) * ATT_HD;
 
     // K and V of block blk (rows past `last` repeat it): the next block of
     // this wave is requested before the current one is multiplied
@@ -692,17 +688,16 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
     h8 kaA[2][4], vrA[2][4];
     if (wv < nblk) load_blk(wv, kaA, vrA);
 
-    // Q^T operands of each head: token tq, dims 32 kk + 8 grp .. +7, scaled,
+    // Q^T operands: token tq, dims 32 kk + 8 grp .. +7, scaled,
     // hi + lo; every wave computes them, wave 0 keeps them in LDS (the block
-    // loop reads one head's at a time, so the accumulators fit the VGPRs)
-    float qs[HPK];   // the scale of head h's scores (undoes the query's power of two)
+    // loop reads them per block)
+    float qs;   // the scale of the scores (undoes the query's power of two)
     const float *q = qkv + (size_t)tq * row_stride;
-#pragma unroll
-    for (int h = 0; h < HPK; h++) {
+    {
         float x[4][8], mx = 0.0f;
 #pragma unroll
         for (int kk = 0; kk < 4; kk++) {
-            const float4 *qp = (const float4 *)(q + (size_t)(g * HPK + h) * ATT_HD + 32 * kk + 8 * grp);
+            const float4 *qp = (const float4 *)(q + (size_t)g * ATT_HD + 32 * kk + 8 * grp);
             const float4 a = qp[0], b = qp[1];
             x[kk][0] = a.x; x[kk][1] = a.y; x[kk][2] = a.z; x[kk][3] = a.w;
             x[kk][4] = b.x; x[kk][5] = b.y; x[kk][6] = b.z; x[kk][7] = b.w;
@@ -716,7 +711,7 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
         int e = 0;
         if (mx > 0.0f && __builtin_isfinite(mx)) (void)frexpf(mx, &e);
         const float up = ldexpf(1.0f, 14 - e);
-        qs[h] = ldexpf(1.0f, e - 14);
+        qs = ldexpf(1.0f, e - 14);
 #pragma unroll
         for (int kk = 0; kk < 4; kk++) {
             h8 qh, ql;
@@ -728,20 +723,19 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
                 ql[i] = (_Float16)(v - (float)hi);
             }
             if (wv == 0) {
-                qop[((h * 4 + kk) * 2) * 64 + l] = qh;
-                qop[((h * 4 + kk) * 2 + 1) * 64 + l] = ql;
+                qop[2 * kk * 64 + l] = qh;
+                qop[(2 * kk + 1) * 64 + l] = ql;
             }
         }
     }
     __syncthreads();   // the Q^T operands are in LDS
-    f4 o[HPK][8];
-    float m[HPK], ls[HPK];
+    f4 o[8];
+    float m, ls;
+    {
+        m = -__builtin_inff();
+        ls = 0.0f;
 #pragma unroll
-    for (int h = 0; h < HPK; h++) {
-        m[h] = -__builtin_inff();
-        ls[h] = 0.0f;
-#pragma unroll
-        for (int dt = 0; dt < 8; dt++) o[h][dt] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int dt = 0; dt < 8; dt++) o[dt] = f4{0.f, 0.f, 0.f, 0.f};
     }
     auto process = [&](uint32_t blk, const h8 (&ka)[2][4], const h8 (&vr)[2][4]) {
         const uint32_t c0 = 32 * blk;
@@ -755,13 +749,12 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
                 *(h4 *)(vt + (8 * n + d) * ATTM_LD + 16 * half + 4 * grp) =
                     h4{vr[half][0][d], vr[half][1][d], vr[half][2][d], vr[half][3][d]};
         wave_lds_order();
-#pragma unroll
-        for (int h = 0; h < HPK; h++) {
+        {
             h8 qh[4], ql[4];
 #pragma unroll
             for (int kk = 0; kk < 4; kk++) {
-                qh[kk] = qop[((h * 4 + kk) * 2) * 64 + l];
-                ql[kk] = qop[((h * 4 + kk) * 2 + 1) * 64 + l];
+                qh[kk] = qop[2 * kk * 64 + l];
+                ql[kk] = qop[(2 * kk + 1) * 64 + l];
             }
             f4 sc[2];
 #pragma unroll
@@ -779,7 +772,7 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
             for (int kt = 0; kt < 2; kt++)
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    sc[kt][r] *= qs[h];
+                    sc[kt][r] *= qs;
                     if (c0 + 16 * kt + 4 * grp + r > tpos) sc[kt][r] = -__builtin_inff();
                     bm = fmaxf(bm, sc[kt][r]);
                 }
@@ -790,14 +783,14 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
             // rescaled in a branch the whole wave skips otherwise.  -inf while
             // none of this wave's blocks so far holds a key of the token's
             // range (a wave's first block may lie past the token).
-            const float mo = m[h];
+            const float mo = m;
             const bool upd = bm > mo + 3.0f;   // -inf + 3 = -inf: a first finite block moves it
             const float mn = upd ? bm : mo;
             const bool none = mn == -__builtin_inff();
             const float cf = upd && mo != -__builtin_inff() ? exp2f(mo - mn) : 1.0f;
             if (__builtin_amdgcn_ballot_w64(cf != 1.0f)) {
 #pragma unroll
-                for (int dt = 0; dt < 8; dt++) o[h][dt] = o[h][dt] * cf;
+                for (int dt = 0; dt < 8; dt++) o[dt] = o[dt] * cf;
             }
             float ps = 0.0f;
             h8 pb, pl;
@@ -812,8 +805,8 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
                     pl[4 * kt + r] = (_Float16)(pp - (float)hi);
                 }
             ps = lanes4_sum(ps);
-            ls[h] = fmaf(ls[h], cf, ps);
-            m[h] = mn;
+            ls = fmaf(ls, cf, ps);
+            m = mn;
             // V^T operands of the 8 dim tiles read first, then the 8 P-hi
             // MFMAs and the 8 P-lo MFMAs (each accumulator takes hi then lo)
             h8 av[8];
@@ -824,14 +817,12 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
                 av[dt] = h8{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
             }
 #pragma unroll
-            for (int dt = 0; dt < 8; dt++) o[h][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[dt], pb, o[h][dt], 0, 0, 0);
+            for (int dt = 0; dt < 8; dt++) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[dt], pb, o[dt], 0, 0, 0);
 #pragma unroll
-            for (int dt = 0; dt < 8; dt++) o[h][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[dt], pl, o[h][dt], 0, 0, 0);
+            for (int dt = 0; dt < 8; dt++) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[dt], pl, o[dt], 0, 0, 0);
         }
     };
-    if constexpr (HPK <= 3) {
-        // two register sets (HPK = 4 would spill: its accumulators take 32
-        // registers more)
+    {   // two register sets
         h8 kaB[2][4], vrB[2][4];
         uint32_t blk = wv;
         while (blk < nblk) {
@@ -843,60 +834,54 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
             process(blk, kaB, vrB);
             blk += ATTM_WAVES;
         }
-    } else {
-        for (uint32_t blk = wv; blk < nblk; blk += ATTM_WAVES) {
-            if (blk != wv) load_blk(blk, kaA, vrA);
-            process(blk, kaA, vrA);
-        }
     }
     // merge the waves: wave w's output rows (token, dims) and its max / sum
-    // per (head, token); a wave without blocks holds max -inf, sum 0
+    // per token; a wave without blocks holds max -inf, sum 0
     __syncthreads();   // every wave is done with its V^T
-#pragma unroll
-    for (int h = 0; h < HPK; h++) {
-        float *orow = mo + ((size_t)(wv * HPK + h) * 16 + n) * ATTM_OLD;
+    {
+        float *orow = mo + ((size_t)wv * 16 + n) * ATTM_OLD;
 #pragma unroll
         for (int dt = 0; dt < 8; dt++)
-            *(float4 *)(orow + 16 * dt + 4 * grp) = make_float4(o[h][dt][0], o[h][dt][1], o[h][dt][2], o[h][dt][3]);
+            *(float4 *)(orow + 16 * dt + 4 * grp) = make_float4(o[dt][0], o[dt][1], o[dt][2], o[dt][3]);
         if (grp == 0) {
-            mml[((wv * HPK + h) * 16 + n) * 2] = m[h];
-            mml[((wv * HPK + h) * 16 + n) * 2 + 1] = ls[h];
+            mml[(wv * 16 + n) * 2] = m;
+            mml[(wv * 16 + n) * 2 + 1] = ls;
         }
     }
     __syncthreads();
-    // per (head, token): the waves' weights exp2(m_w - M) and the output
+    // per token: the waves' weights exp2(m_w - M) and the output
     // scale 1 / (PS L), once (L summed over the waves in order)
-    if (threadIdx.x < HPK * 16) {
-        const uint32_t ht = threadIdx.x, h = ht % HPK, t = ht / HPK;
+    if (threadIdx.x < 16) {
+        const uint32_t t = threadIdx.x;
         float M = -__builtin_inff();
 #pragma unroll
-        for (uint32_t w = 0; w < ATTM_WAVES; w++) M = fmaxf(M, mml[((w * HPK + h) * 16 + t) * 2]);
+        for (uint32_t w = 0; w < ATTM_WAVES; w++) M = fmaxf(M, mml[(w * 16 + t) * 2]);
         float L = 0.0f;
 #pragma unroll
         for (uint32_t w = 0; w < ATTM_WAVES; w++) {
-            const float c = safe_scale(mml[((w * HPK + h) * 16 + t) * 2], M);   // 0 for a wave without rows
-            L = fmaf(mml[((w * HPK + h) * 16 + t) * 2 + 1], c, L);
-            mcw[ht * (ATTM_WAVES + 1) + w] = c;
+            const float c = safe_scale(mml[(w * 16 + t) * 2], M);   // 0 for a wave without rows
+            L = fmaf(mml[(w * 16 + t) * 2 + 1], c, L);
+            mcw[t * (ATTM_WAVES + 1) + w] = c;
         }
-        mcw[ht * (ATTM_WAVES + 1) + ATTM_WAVES] = (1.0f / ATTM_PS) / L;
+        mcw[t * (ATTM_WAVES + 1) + ATTM_WAVES] = (1.0f / ATTM_PS) / L;
     }
     __syncthreads();
     // four dims a thread: the waves' outputs weighted and added in wave order
-    const size_t qd = (size_t)gridDim.x * HPK * ATT_HD;
-    for (uint32_t i = threadIdx.x; i < HPK * 16 * ATT_HD / 4; i += 64 * ATTM_WAVES) {
-        const uint32_t d = 4 * (i % (ATT_HD / 4)), ht = i / (ATT_HD / 4), h = ht % HPK, t = ht / HPK;   // dims fastest
+    const size_t qd = (size_t)gridDim.x * ATT_HD;
+    for (uint32_t i = threadIdx.x; i < 16 * ATT_HD / 4; i += 64 * ATTM_WAVES) {
+        const uint32_t d = 4 * (i % (ATT_HD / 4)), t = i / (ATT_HD / 4);   // dims fastest
         const uint32_t tk = tb * 16 + t;
-        const float *cw = mcw + ht * (ATTM_WAVES + 1);
+        const float *cw = mcw + t * (ATTM_WAVES + 1);
         f4 O = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (uint32_t w = 0; w < ATTM_WAVES; w++) {
             const float c = cw[w];
-            const f4 ow = *(const f4 *)(mo + ((size_t)(w * HPK + h) * 16 + t) * ATTM_OLD + d);
+            const f4 ow = *(const f4 *)(mo + ((size_t)w * 16 + t) * ATTM_OLD + d);
 #pragma unroll
             for (int e = 0; e < 4; e++) O[e] = fmaf(ow[e], c, O[e]);
         }
         if (tk < rows) {
-            const size_t oi = (size_t)tk * qd + (size_t)(g * HPK + h) * ATT_HD + d;
+            const size_t oi = (size_t)tk * qd + (size_t)g * ATT_HD + d;
             const float sc = cw[ATTM_WAVES];
             f4 v;
 #pragma unroll
@@ -914,20 +899,9 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
 template <int HPK>
 static void go_attn_prefill(const float *qkv, uint32_t row_stride, uint32_t rows, const uint16_t *kc,
                             const uint16_t *vc, void *out, bool out_f16, uint32_t pos0, uint32_t n_kv_heads,
-                            float qscale, hipStream_t s, uint32_t hsplit = 1)
+                            float qscale, hipStream_t s)
 {
     const uint32_t kv_stride = n_kv_heads * ATT_HD;
-    if constexpr (HPK <= 4) {   // the matrix-core form (its accumulators take 32 registers per head)
-        const dim3 grid(n_kv_heads * hsplit, (rows + 15) / 16);
-        static_assert(AttmLds<4>::BYTES <= 160 * 1024, "LDS per workgroup");
-        if (out_f16)
-            hipLaunchKernelGGL((attn_prefill_mfma_kernel<HPK, true>), grid, dim3(64 * ATTM_WAVES), 0, s, qkv,
-                               row_stride, kc, vc, out, rows, pos0, kv_stride, qscale, hsplit);
-        else
-            hipLaunchKernelGGL((attn_prefill_mfma_kernel<HPK, false>), grid, dim3(64 * ATTM_WAVES), 0, s, qkv,
-                               row_stride, kc, vc, out, rows, pos0, kv_stride, qscale, hsplit);
-        return;
-    }
     if (out_f16)
         hipLaunchKernelGGL((attn_prefill_kernel<HPK, true>), dim3(n_kv_heads, rows), dim3(256), 0, s, qkv, row_stride,
                            kc, vc, out, pos0, kv_stride, qscale);
@@ -942,20 +916,33 @@ hipError_t launch_attention_prefill(const float *qkv, uint32_t row_stride, uint3
 {
     if (rows == 0) return hipSuccess;
     const float qscale = (float)(1.4426950408889634 / sqrt((double)ATT_HD));   // log2(e) / sqrt(head_dim)
-    // a short prompt's workgroups (KV head, 16 tokens) leave CUs idle: then
-    // one workgroup per query head (the same arithmetic per head, bitwise
-    // the grouped form; 128 rows x 8 x 3 heads: 7.6 instead of 12.2 us),
-    // else the KV group's heads share every K/V block in one workgroup
-    // (512 rows: 22.4 against 30.8 us split)
-    const uint64_t tgroups = (rows + 15) / 16;
-    if (heads_per_kv > 1 && heads_per_kv <= 4 && (uint64_t)n_kv_heads * heads_per_kv * tgroups <= device_cu_count()) {
-        go_attn_prefill<1>(qkv, row_stride, rows, kc, vc, out, out_f16, pos0, n_kv_heads, qscale, s, heads_per_kv);
+    // Up to 4 query heads a KV head.  Where one workgroup per query head and 16
+    // tokens covers the CUs at most once, that form (128 rows of 8 x 3 heads 9.7
+    // us against 12.9); beyond, the form whose waves share each K/V tile (256
+    // rows 14.2 us against 18.1, 2,000 rows 76 against 156), with 64 query rows
+    // a workgroup while those are at most two to a CU (1,000 rows of 8 x 3
+    // heads 33 us against 36, 2,000 of 8 x 1 40 against 57), else 128 (2,000 of
+    // 8 x 3 76 against 89, which reads each key half as often).
+    const uint32_t cus = device_cu_count();
+    if (heads_per_kv <= 4) {
+        if ((uint64_t)n_kv_heads * heads_per_kv * ((rows + 15) / 16) > cus) {
+            const uint64_t wgs = (uint64_t)n_kv_heads * (((uint64_t)rows * heads_per_kv + 63) / 64);
+            return launch_attn_flash(qkv, row_stride, rows, kc, vc, out, out_f16, pos0, n_kv_heads, heads_per_kv, qscale,
+                                     wgs <= 2 * cus ? 4 : 2, s);
+        }
+        const dim3 grid(n_kv_heads * heads_per_kv, (rows + 15) / 16);
+        const uint32_t kv_stride = n_kv_heads * ATT_HD;
+        if (out_f16)
+            hipLaunchKernelGGL(attn_prefill_mfma_kernel<true>, grid, dim3(64 * ATTM_WAVES), 0, s, qkv, row_stride, kc, vc,
+                               out, rows, pos0, kv_stride, qscale, heads_per_kv);
+        else
+            hipLaunchKernelGGL(attn_prefill_mfma_kernel<false>, grid, dim3(64 * ATTM_WAVES), 0, s, qkv, row_stride, kc, vc,
+                               out, rows, pos0, kv_stride, qscale, heads_per_kv);
         return hipGetLastError();
     }
 #define RRR_ATTP_CASE(H) \
     case H: go_attn_prefill<H>(qkv, row_stride, rows, kc, vc, out, out_f16, pos0, n_kv_heads, qscale, s); break;
     switch (heads_per_kv) {
-        RRR_ATTP_CASE(1) RRR_ATTP_CASE(2) RRR_ATTP_CASE(3) RRR_ATTP_CASE(4)
         RRR_ATTP_CASE(5) RRR_ATTP_CASE(6) RRR_ATTP_CASE(7) RRR_ATTP_CASE(8)
     default: return hipErrorInvalidValue;
     }

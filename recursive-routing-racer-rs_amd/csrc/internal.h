@@ -131,6 +131,11 @@ hipError_t launch_attention(const float *q, const uint16_t *kc, const uint16_t *
 hipError_t launch_attention_prefill(const float *qkv, uint32_t row_stride, uint32_t rows, const uint16_t *kc,
                                     const uint16_t *vc, void *out, bool out_f16, uint32_t pos0, uint32_t n_kv_heads,
                                     uint32_t heads_per_kv, hipStream_t s);
+// The same with the K/V tiles shared by a workgroup's waves (attn_flash.hip),
+// kq = 2 or 4 waves to a row group's keys.
+hipError_t launch_attn_flash(const float *qkv, uint32_t row_stride, uint32_t rows, const uint16_t *kc,
+                             const uint16_t *vc, void *out, bool out_f16, uint32_t pos0, uint32_t n_kv, uint32_t hpk,
+                             float qscale, uint32_t kq, hipStream_t s);
 // Prefill dequant-GEMM (gemm.hip): X is M x K bf16 or f16 bits; Y = X . W^T,
 // or Y += X . W^T with accumulate; with rscale, row m of the product is
 // multiplied by rscale[m] (a power of two: exact) first.  ws (ws_bytes, may
