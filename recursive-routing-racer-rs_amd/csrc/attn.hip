@@ -83,12 +83,17 @@ hipError_t launch_rope_kv_store(float *qkv, const RopeArgs &r, uint16_t *kc, uin
 // gemm_splitk_reduce adds them), then the rope_kv_store of the row: every
 // element of qkv, and the caches, end bit for bit as after the reduction
 // followed by rope_kv_store_kernel.  Rows m >= rows (the GEMM's padding rows)
-// get the plain sums (SS = S, 2..8: a quad's partials are all requested
-// before the first add).  Four elements (two pairs) a thread; the launcher
-// requires q_dim, kv_stride and row_stride (= the GEMM's N) % 4 == 0, so a
-// quad never straddles the Q, K and V parts.
+// get the plain sums.  A thread takes two quads of elements (two pairs each) a
+// pass, and the launcher as many threads as make one pass of the row up to 8,192
+// elements: bound by latency at a few rows (the partials' round trip and the
+// coefficients' powf and sincosf, which the requests now overlap), by HBM at
+// many.  128 rows of 5,120 at three splits 7.0 -> 4.9 us against 256 threads and
+// five dependent passes, 512 rows 11.2 in both.  The launcher requires q_dim,
+// kv_stride and row_stride (= the GEMM's N) % 4 == 0, so a quad never straddles
+// the Q, K and V parts.
+constexpr uint32_t srk_threads(int SS) { return SS <= 6 ? 1024u : 512u; }   // registers for the partials in flight
 template <int SS>
-__global__ __launch_bounds__(256) void splitk_rope_kv_store_kernel(const float *__restrict__ ws, uint32_t M,
+__global__ __launch_bounds__(srk_threads(SS)) void splitk_rope_kv_store_kernel(const float *__restrict__ ws, uint32_t M,
                                                                    float *__restrict__ qkv, RopeArgs r, uint32_t rows,
                                                                    uint32_t *__restrict__ kc, uint32_t *__restrict__ vc,
                                                                    uint32_t lds_coef)
@@ -97,11 +102,22 @@ __global__ __launch_bounds__(256) void splitk_rope_kv_store_kernel(const float *
     const uint32_t N = r.row_stride, m = blockIdx.y, half_rope = r.rope_dim / 2;
     const uint32_t pos = r.pos + m, qh = r.n_heads * r.head_dim;
     const bool live = m < rows;
-    const uint64_t mn = (uint64_t)M * N;
-    const float *src = ws + (uint64_t)m * N;
+    const uint32_t mn4 = M * N * 4, TH = blockDim.x;              // bytes of one split's partials
     float *dst = qkv + (uint64_t)m * N;
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(ws, (uint64_t)SS * mn4);
+    u32x4 p[2][SS];
+    auto request = [&](uint32_t c0) {   // quads c0 + 4 t and c0 + 4 (TH + t); past the row: no request
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const uint32_t c = c0 + 4 * (i * TH + threadIdx.x);
+#pragma unroll
+            for (int k = 0; k < SS; k++) p[i][k] = bload16_so(rw, c < N ? (m * N + c) * 4 : RRR_OOB, k * mn4);
+        }
+    };
+    request(0);
+    __builtin_amdgcn_sched_barrier(0);
     if (lds_coef && live) {
-        for (uint32_t j = threadIdx.x; j < half_rope; j += 256) rope_coef(j, pos, r, cf[2 * j], cf[2 * j + 1]);
+        for (uint32_t j = threadIdx.x; j < half_rope; j += TH) rope_coef(j, pos, r, cf[2 * j], cf[2 * j + 1]);
         __syncthreads();
     }
     auto coef = [&](uint32_t j, float &cs, float &ss) {
@@ -112,14 +128,12 @@ __global__ __launch_bounds__(256) void splitk_rope_kv_store_kernel(const float *
             rope_coef(j, pos, r, cs, ss);
         }
     };
-    for (uint32_t c = 4 * (blockIdx.x * 256 + threadIdx.x); c < N; c += 4 * gridDim.x * 256) {
-        float4 p[SS];
-#pragma unroll
-        for (int k = 0; k < SS; k++) p[k] = *(const float4 *)(src + k * mn + c);
-        float4 v = p[0];
+    auto quad = [&](uint32_t c, const u32x4 (&w)[SS]) {
+        float4 v = u2f4(w[0]);
 #pragma unroll
         for (int k = 1; k < SS; k++) {
-            v.x += p[k].x; v.y += p[k].y; v.z += p[k].z; v.w += p[k].w;
+            const float4 u = u2f4(w[k]);
+            v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
         }
         if (live) {
             float x[4] = {v.x, v.y, v.z, v.w};
@@ -160,6 +174,14 @@ __global__ __launch_bounds__(256) void splitk_rope_kv_store_kernel(const float *
             v = make_float4(x[0], x[1], x[2], x[3]);
         }
         *(float4 *)(dst + c) = v;
+    };
+    for (uint32_t c0 = 0; c0 < N; c0 += 8 * TH) {
+        if (c0) request(c0);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const uint32_t c = c0 + 4 * (i * TH + threadIdx.x);
+            if (c < N) quad(c, p[i]);
+        }
     }
 }
 
@@ -176,9 +198,10 @@ hipError_t launch_splitk_rope_kv_store(const float *ws, uint32_t S, uint32_t M, 
     if (!splitk_rope_kv_store_supported(r)) return hipErrorNotSupported;
     const size_t lds = (size_t)r.rope_dim * 4;
     const uint32_t lds_coef = lds <= 32 * 1024 ? 1u : 0u;
+    const uint32_t th = min(srk_threads((int)S), (r.row_stride + 511) / 512 * 64);   // two quads a thread
 #define RRR_SRK_CASE(K)                                                                                          \
     case K:                                                                                                       \
-        hipLaunchKernelGGL(splitk_rope_kv_store_kernel<K>, dim3(1, M), dim3(256), lds_coef ? lds : 0, s, ws, M, qkv, \
+        hipLaunchKernelGGL(splitk_rope_kv_store_kernel<K>, dim3(1, M), dim3(th), lds_coef ? lds : 0, s, ws, M, qkv, \
                            r, rows, (uint32_t *)kc, (uint32_t *)vc, lds_coef);                                      \
         break;
     switch (S) {
