@@ -81,6 +81,7 @@ hipError_t launch_rmsnorm(const float *x, const float *g, float *y, uint32_t row
 hipError_t launch_silu_gate(const float *gu, float *mid, uint32_t rows, uint32_t F, hipStream_t s);
 hipError_t launch_residual_add(const float *a, const float *b, float *out, uint32_t n, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t *p, uint64_t n_words, uint32_t v, hipStream_t s);
+hipError_t launch_copy_f32(const float *src, float *dst, uint32_t n, hipStream_t s);
 // Transposed-chunk logits (layout 1).  gamma != nullptr fuses the RMSNorm.
 hipError_t launch_logits_chunked(const float *x, const float *gamma, float eps, const float *E,
                                  float *y, uint32_t K, uint32_t V, uint32_t chunk, hipStream_t s);

@@ -430,6 +430,21 @@ hipError_t launch_fill_u32(uint32_t *p, uint64_t n, uint32_t v, hipStream_t s)
     return hipGetLastError();
 }
 
+// n floats from src to dst, either in pinned host memory (the staging of
+// rrr_matmul_kquant); both 16-byte aligned.
+__global__ __launch_bounds__(256) void copy_f32_kernel(const float *__restrict__ src, float *__restrict__ dst, uint32_t n)
+{
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n / 4) ((float4 *)dst)[i] = ((const float4 *)src)[i];
+    if (i < n % 4) dst[n / 4 * 4 + i] = src[n / 4 * 4 + i];
+}
+
+hipError_t launch_copy_f32(const float *src, float *dst, uint32_t n, hipStream_t s)
+{
+    hipLaunchKernelGGL(copy_f32_kernel, dim3(n / 1024 + 1), dim3(256), 0, s, src, dst, n);
+    return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------
 // Logits over the reference's transposed chunks (phi4.rs:874-893):
 // chunk c holds n_c = min(chunk, V - c*chunk) vocab rows as B_c[d*n_c + v].
