@@ -694,6 +694,12 @@ static int logits_common(rrr_ctx *ctx, const rrr_buf *x, const rrr_buf *gamma, f
         a.K = K;
         a.N = V;
         a.M = 1;
+        // Q6_K: the GEMV leaves the argmax's candidates, one launch less
+        if (token && gamma) {
+            a.cand = ctx->scratch;
+            const hipError_t e = launch_gemv_argmax(a, token, ctx->stream);
+            if (e != hipErrorNotSupported) return finish(ctx, e, what);
+        }
         return finish(ctx, then_argmax(launch_gemv(a, gamma ? ACT_RMSNORM : ACT_PLAIN, ctx->stream)), what);
     }
     if (chunk == 0) return fail(RRR_ERR_INVALID_ARG, "%s: chunk must be positive", what);

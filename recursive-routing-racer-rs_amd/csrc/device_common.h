@@ -438,3 +438,26 @@ __device__ __forceinline__ float silu_f(float g) { return g / (1.0f + expf(-g));
 // reference's GPU shader uses a relaxed exp as well).  The standalone
 // silu_gate keeps silu_f.
 __device__ __forceinline__ float silu_fast(float g) { return __fdividef(g, 1.0f + __expf(-g)); }
+
+// A candidate of the argmax rule of phi4.rs:1172-1183 (value -inf, index 0 at
+// the start, replaced only by a strictly greater value).
+struct Cand { float v; uint32_t i; };
+
+__device__ __forceinline__ Cand better(Cand a, Cand b)
+{
+    // a precedes b in index order whenever both are live candidates
+    if (b.v > a.v || (b.v == a.v && b.i < a.i)) return b;
+    return a;
+}
+
+__device__ __forceinline__ Cand wave_best(Cand c)
+{
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        Cand d;
+        d.v = __shfl_xor(c.v, o, 64);
+        d.i = __shfl_xor(c.i, o, 64);
+        c = better(c, d);
+    }
+    return c;
+}

@@ -11,6 +11,13 @@ __global__ __launch_bounds__(1024) void gemv_mq_kernel(GemvArgs a, uint32_t ntil
     mq_body<Q, BPW, ACT, MULTI, TR, PAIR, ROPE, ST>(a, ntiles, tr);
 }
 
+// The logits form: fused RMSNorm, argmax candidates in the epilogue.
+template <class Q, int BPW>
+__global__ __launch_bounds__(1024) void gemv_mq_argmax_kernel(GemvArgs a, uint32_t ntiles, uint32_t tr)
+{
+    mq_body<Q, BPW, ACT_RMSNORM, true, 16, false, false, false, 1, true>(a, ntiles, tr);
+}
+
 // The multi-token form, MT rows of x per weight stream, in workgroups of at
 // most NTH threads (768 = 12 waves leaves 168 registers a lane where 1024
 // threads leave 128, which MT = 4 and 8 exceed).
@@ -27,18 +34,24 @@ struct MqShape {
 
 // Super-blocks per wave and waves per workgroup (at least 4; waves past the
 // last super-block only encode).
-// Up to one workgroup per CU, each taking its tiles as far as its row
-// partials fit in LDS.  Tiles split evenly over the CUs (a wave issues only
-// the load slots its tile height needs, so short tiles cost no empty loads).
+// Up to one workgroup per CU (two of 4 waves, K <= 1024, where N has more
+// than 16 rows a CU: the loads in flight of 4 waves leave the memory idle,
+// Q6_K 1024 x 128256 28.6 -> 21.2 us, Q4_K 1024 x 8192 4.9 -> 4.6 us; four of
+// 4 waves 22.1, two of 8 waves 42.0 for 36.6 us), each taking its tiles as far
+// as its row partials fit in LDS.  Tiles split evenly over the CUs (a wave
+// issues only the load slots its tile height needs, so short tiles cost no
+// empty loads).
 template <class Q, int BPW>
-static void mq_plan(const GemvArgs &a, uint32_t &W, uint32_t &grid, size_t &lds, uint32_t &tr, uint32_t &ntiles)
+static void mq_plan(const GemvArgs &a, uint32_t &W, uint32_t &grid, size_t &lds, uint32_t &tr, uint32_t &ntiles,
+                    uint32_t per_cu = 2)
 {
     using G = MwGeom<Q, BPW>;
     W = mq_waves(a.K, BPW);
     const size_t fixed = W * G::BYTES + 64;
-    const uint32_t per_max = (uint32_t)((160 * 1024 - fixed) / (W * 64));
+    const uint32_t cus = device_cus(), share = W == 4 && a.N > 16 * cus ? per_cu : 1u;
+    const uint32_t per_max = (uint32_t)((160 * 1024 / share - fixed) / (W * 64));
     uint32_t per;
-    mq_tiles(a.N, device_cus(), per_max, 1u, tr, ntiles, per);
+    mq_tiles(a.N, cus * share, per_max, 1u, tr, ntiles, per);
     grid = (ntiles + per - 1) / per;
     lds = fixed + (size_t)per * W * 64;
 }
@@ -102,7 +115,7 @@ static hipError_t go_mq_rope(const GemvArgs &a, hipStream_t s)
 {
     uint32_t W, grid, tr, ntiles;
     size_t lds;
-    mq_plan<Q, BPW>(a, W, grid, lds, tr, ntiles);
+    mq_plan<Q, BPW>(a, W, grid, lds, tr, ntiles, 1);   // as many even heights as one workgroup a CU gives
     if (tr % 2) return hipErrorNotSupported;
     lds += 4 * (size_t)a.rope.rope_dim;   // the rotation coefficients
     if (lds > 160 * 1024) return hipErrorNotSupported;
@@ -123,6 +136,17 @@ static hipError_t go_mq_rope(const GemvArgs &a, hipStream_t s)
                                lds, s, a, ntiles, tr);
     }
     return hipGetLastError();
+}
+
+template <class Q, int BPW>
+static hipError_t go_mq_argmax(const GemvArgs &a, uint32_t *token, hipStream_t s)
+{
+    uint32_t W, grid, tr, ntiles;
+    size_t lds;
+    mq_plan<Q, BPW>(a, W, grid, lds, tr, ntiles);
+    if (grid > ARGMAX_WG) return hipErrorNotSupported;
+    hipLaunchKernelGGL((gemv_mq_argmax_kernel<Q, BPW>), dim3(grid), dim3(64 * W), lds, s, a, ntiles, tr);
+    return launch_argmax_candidates(a.cand, grid, token, s);
 }
 
 template <class Q, int ACT, bool ST>
@@ -244,6 +268,12 @@ hipError_t launch_gemv_mfma(const GemvArgs &a, uint32_t act, hipStream_t s)
     case T_Q6_K: return go_mq_act<MqQ6K>(a, act, s);
     default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_gemv_argmax(const GemvArgs &a, uint32_t *token, hipStream_t s)
+{
+    if (a.type != T_Q6_K || a.residual || !gemv_mfma_supported(a)) return hipErrorNotSupported;
+    return a.K <= 16 * 256 ? go_mq_argmax<MqQ6K, 1>(a, token, s) : go_mq_argmax<MqQ6K, 2>(a, token, s);
 }
 
 // The launch launch_gemv_mfma makes for `a` (plain and pair forms; not the

@@ -321,16 +321,22 @@ __device__ __forceinline__ uint64_t phase_stamp(float dep)
     return t;
 }
 
+// AM: the workgroup's candidate for the argmax of the rows, from the threads
+// that write them, to a.cand[block]; one small launch reduces the candidates.
+// That launch costs 2 us where the two of rrr_argmax_f32 cost 4; reducing them
+// in the last workgroup to arrive was slower, its counter taking 12 ns per
+// workgroup (256 of them: 4.5 us).
 // MT > 1: the multi-token form (plain activations; a.M <= MT tokens, rows m
 // of x at x + m K, outputs at y + m N; tokens past a.M read the last row and
 // store nothing).
 template <class Q, int BPW, int ACT, bool MULTI, int TR = 16, bool PAIR = false, bool ROPE = false,
-          bool STAMPS = false, int MT = 1>
+          bool STAMPS = false, int MT = 1, bool AM = false>
 __device__ __forceinline__ void mq_body(const GemvArgs &a, uint32_t ntiles, uint32_t tr)
 {
     extern __shared__ float smem[];
     using G = MwGeom<Q, BPW, MT>;
     static_assert(TR >= 1 && TR <= 16, "tile rows");
+    static_assert(!AM || (MULTI && MT == 1 && !PAIR && !ROPE && !STAMPS), "argmax epilogue on a plain row layout");
     static_assert(MT == 1 || (ACT == ACT_PLAIN && !PAIR && !ROPE && !STAMPS), "multi-token form: plain rows");
     constexpr int SB = (TR + (int)G::RPS - 1) / (int)G::RPS;     // load slots of one block
     // A operands in registers, except in the persistent two-block form, whose
@@ -657,6 +663,25 @@ __device__ __forceinline__ void mq_body(const GemvArgs &a, uint32_t ntiles, uint
             mark(14, 0.0f);
             mark_flush();
         }
+        return;
+    }
+    if constexpr (AM) {
+        Cand c = {-__builtin_inff(), 0u};
+        for (uint32_t i = t; i < ntl * 16; i += NT) {
+            const uint32_t tl = i >> 4, r = i & 15, row = (tile0 + tl * GR) * tr + r;   // ascending
+            if (r < tr && row < a.N) {
+                const float v = waves_sum(part + tl * W * 16 + r, W);
+                a.y[row] = v;
+                if (v > c.v) c = Cand{v, row};   // NaN and -inf never win
+            }
+        }
+        c = wave_best(c);
+        Cand *sm = (Cand *)smem;   // wave 0's region, read by nobody past the barrier above
+        if (lane == 0) sm[wave] = c;
+        __syncthreads();
+        if (wave) return;
+        c = wave_best(lane < W ? sm[lane] : Cand{-__builtin_inff(), 0u});
+        if (lane == 0) ((Cand *)a.cand)[blockIdx.x] = c;
         return;
     }
     for (uint32_t i = t; i < ntl * MT * 16; i += NT) {

@@ -45,6 +45,7 @@ struct GemvArgs {
     uint32_t rope_on;
     RopeArgs rope;
     uint32_t *kc, *vc;
+    void *cand;           // launch_gemv_argmax: one candidate per workgroup (at most ARGMAX_WG)
     uint64_t *stamps;     // phase timestamps of the stamped launch (rrr_probe_gemv_phases), else unused
 };
 
@@ -60,6 +61,9 @@ hipError_t launch_gemv(const GemvArgs &a, uint32_t act, hipStream_t s);
 // int8-MFMA batch-1 K-quant GEMV (gemv_mfma.hip)
 bool gemv_mfma_supported(const GemvArgs &a);
 hipError_t launch_gemv_mfma(const GemvArgs &a, uint32_t act, hipStream_t s);
+// The fused-RMSNorm GEMV of Q6_K rows, then the argmax of y to *token;
+// hipErrorNotSupported (nothing launched) for what it does not take.
+hipError_t launch_gemv_argmax(const GemvArgs &a, uint32_t *token, hipStream_t s);
 // the same launch with phase timestamps into a.stamps (16 u64 per wave of
 // each workgroup); returns the grid and the waves per workgroup
 hipError_t launch_gemv_mfma_stamped(const GemvArgs &a, uint32_t act, hipStream_t s, uint32_t &grid, uint32_t &waves);
@@ -97,7 +101,9 @@ hipError_t launch_logits_split(const float *x, const float *gamma, float eps, co
                                uint32_t V, uint32_t chunk, float *part, uint32_t *counters, uint32_t *token,
                                hipStream_t s);
 // Argmax: `partials` holds at least argmax_partials_bytes() bytes.
+constexpr uint32_t ARGMAX_WG = 1024;   // candidates
 uint64_t argmax_partials_bytes();
+hipError_t launch_argmax_candidates(const void *partials, uint32_t n, uint32_t *out, hipStream_t s);
 hipError_t launch_argmax(const float *v, uint32_t n, void *partials, uint32_t *out, hipStream_t s);
 // RoPE + f16 KV store (attn.hip): the rope_kv_store / kv_store pipelines.
 // rows consecutive tokens at positions pos .. pos + rows - 1

@@ -541,27 +541,6 @@ hipError_t launch_logits_chunked(const float *x, const float *gamma, float eps, 
 // start from (value -inf, index 0), replace only on strictly greater, so the
 // first maximal index wins and NaN never wins.  Pass 1: one candidate per
 // workgroup; pass 2: one workgroup reduces the candidates in index order.
-struct Cand { float v; uint32_t i; };
-
-__device__ __forceinline__ Cand better(Cand a, Cand b)
-{
-    // a precedes b in index order whenever both are live candidates
-    if (b.v > a.v || (b.v == a.v && b.i < a.i)) return b;
-    return a;
-}
-
-__device__ __forceinline__ Cand wave_best(Cand c)
-{
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-        Cand d;
-        d.v = __shfl_xor(c.v, o, 64);
-        d.i = __shfl_xor(c.i, o, 64);
-        c = better(c, d);
-    }
-    return c;
-}
-
 __device__ Cand block_best(Cand c, Cand *sm)
 {
     c = wave_best(c);
@@ -739,8 +718,6 @@ hipError_t launch_logits_split(const float *x, const float *gamma, float eps, co
     return hipGetLastError();
 }
 
-constexpr uint32_t ARGMAX_WG = 1024;
-
 __global__ __launch_bounds__(256) void argmax_pass1(const float *__restrict__ v, uint32_t n, Cand *part)
 {
     __shared__ Cand sm[4];
@@ -770,7 +747,12 @@ hipError_t launch_argmax(const float *v, uint32_t n, void *partials, uint32_t *o
     if (wg > ARGMAX_WG) wg = ARGMAX_WG;
     if (wg == 0) wg = 1;
     hipLaunchKernelGGL(argmax_pass1, dim3(wg), dim3(256), 0, s, v, n, (Cand *)partials);
-    hipLaunchKernelGGL(argmax_pass2, dim3(1), dim3(256), 0, s, (const Cand *)partials, wg, out);
+    return launch_argmax_candidates(partials, wg, out, s);
+}
+
+hipError_t launch_argmax_candidates(const void *partials, uint32_t n, uint32_t *out, hipStream_t s)
+{
+    hipLaunchKernelGGL(argmax_pass2, dim3(1), dim3(256), 0, s, (const Cand *)partials, n, out);
     return hipGetLastError();
 }
 
