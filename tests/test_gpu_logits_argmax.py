@@ -1,76 +1,128 @@
-"""rrr_logits_rmsnorm_argmax on Q6_K rows: the logits of rrr_logits_rmsnorm bit for bit and the first index of their
-maximum, from one row to several tiles a workgroup, either side of a wave's one and two super-blocks and past the widest
-K of the epilogue; with ties across workgroups, without a live candidate, eager and in a replayed graph.  And the GEMV
-below it where two workgroups share a CU."""
+"""The logits with their argmax in one call (rrr_logits_rmsnorm_argmax).
+
+On the reference's transposed chunks the argmax runs inside the split-K
+logits launch: the last workgroup of each 256-entry slab reduces the slab to
+its (max, first index), and the last slab to finish reduces the slabs'
+candidates.  Checked on the same inputs: the logits are bitwise those of
+rrr_logits_rmsnorm, and the index is both rrr_argmax_f32's on those logits
+and the sequential rule of phi4.rs:1172-1183 applied on the host (start from
+(-inf, 0), replace only on strictly greater: the first maximal index wins,
+NaN never wins) -- with ties planted across chunks and inside one slab, a row
+whose logit is NaN and rows whose logit is +inf.  Repeated calls and graph
+replays return the same index (the arrival counters return to zero).
+"""
 import numpy as np
 import pytest
 
-import rrr_hip as rrr
+import oracle.oracle as orc
+import rrr_hip
 from rrr_hip import synth
 
 pytestmark = pytest.mark.gpu
-EPS = 1e-5
+
+K = 3072
 
 
-@pytest.mark.parametrize("K,V", [(256, 1), (256, 17), (512, 4097), (1024, 32064), (3072, 1000), (3072, 32064), (4096, 4099),
-                                 (4352, 5000), (8192, 2561), (8192, 70000), (8448, 300)])
-@pytest.mark.parametrize("same", [False, True])
-def test_token_is_first_max_of_the_same_logits(K, V, same):
-    raw = np.frombuffer(synth.weight(61, 1, rrr.Q6_K, K, V), np.uint8)
-    if same:   # rows repeat every 7: the maximum is in many workgroups
-        rows = raw.reshape(V, -1)
-        raw = np.ascontiguousarray(rows[np.arange(V) % 7]).reshape(-1)
-    with rrr.Context(0) as ctx:
-        E, g = ctx.weight_upload(rrr.Q6_K, K, V, raw), ctx.alloc(K * 4)
-        x, y, y2 = ctx.alloc(K * 4), ctx.alloc((V + 4) * 4), ctx.alloc(V * 4)
-        token = ctx.alloc(4)
-        ctx.upload(g, 1.0 + 0.1 * synth.normal_f32(62, 1, K))
-        issue = lambda t=token: ctx.logits_rmsnorm_argmax(x, g, EPS, E, y, K, V, t, rrr.LOGITS_Q6K, 0)
-        ctx.upload(x, synth.normal_f32(62, 2, K))
-        ctx.graph_begin()
-        issue()
-        graph = ctx.graph_end()
-        for i, run in enumerate([issue, graph.launch, issue, graph.launch, graph.launch]):
-            ctx.upload(x, synth.normal_f32(63, i, K))
-            ctx.fill_u32(y, 0x7F7F7F7F)
-            ctx.fill_u32(token, 0xFFFFFFFF)
-            run()
-            got = ctx.download(y, np.uint32)
-            ctx.logits_rmsnorm(x, g, EPS, E, y2, K, V, rrr.LOGITS_Q6K, 0)
-            ref = ctx.download(y2)
-            assert np.array_equal(got[:V], ref.view(np.uint32)) and np.all(got[V:] == 0x7F7F7F7F)
-            assert ctx.download(token, np.uint32)[0] == np.argmax(ref)
-        graph.destroy()
-        for bad in (0.0, np.nan):   # all logits zero: index 0; all NaN: no candidate, index 0
-            v = synth.normal_f32(63, 9, K) * (0.0 if bad == 0.0 else 1.0)
-            v[K // 2] = bad
-            ctx.upload(x, v.astype(np.float32))
-            ctx.fill_u32(token, 0xFFFFFFFF)
-            issue()
-            assert ctx.download(token, np.uint32)[0] == 0
-        # a token stored over one of the logits: the token is what stays
-        ctx.upload(x, synth.normal_f32(63, 10, K))
-        issue()
-        want = ctx.download(token, np.uint32)[0]
-        issue(ctx.view(y, (V // 2) * 4, 4))
-        assert ctx.download(y, np.uint32)[V // 2] == want
+def host_argmax(v):
+    """The sequential rule, vectorised: NaN never wins, the first maximum does."""
+    ok = ~np.isnan(v)
+    if not ok.any():
+        return 0
+    m = v[ok].max()
+    if m == -np.inf:
+        return 0
+    return int(np.flatnonzero(ok & (v == m))[0])
 
 
-@pytest.mark.parametrize("qtype,K,N", [(12, 1024, 4097), (13, 256, 8193), (14, 1024, 16397), (14, 768, 20480)])
-def test_two_workgroups_a_cu_give_the_bits_of_one(qtype, K, N):
-    rows = np.frombuffer(synth.weight(64, 1, qtype, K, N), np.uint8).reshape(N, -1)
-    with rrr.Context(0) as ctx:
-        x, y, g = ctx.alloc(K * 4), ctx.alloc((N + 4) * 4), ctx.alloc(K * 4)
-        ctx.upload(x, synth.normal_f32(65, 1, K))
-        ctx.upload(g, 1.0 + 0.1 * synth.normal_f32(65, 2, K))
-        W = ctx.weight_upload(qtype, K, N, rows.reshape(-1))
-        part = ctx.alloc(4096 * 4)
-        ctx.fill_u32(y, 0x7F7F7F7F)
-        ctx.gemv_rmsnorm(x, g, EPS, W, qtype, y, K, N)
-        got = ctx.download(y, np.uint32)
-        assert np.all(got[N:] == 0x7F7F7F7F)
-        for r in range(0, N, 4096):   # 16 rows a CU: one workgroup each
-            n = min(4096, N - r)
-            Wr = ctx.weight_upload(qtype, K, n, np.ascontiguousarray(rows[r:r + n]).reshape(-1))
-            ctx.gemv_rmsnorm(x, g, EPS, Wr, qtype, part, K, n)
-            assert np.array_equal(got[r:r + n], ctx.download(part, np.uint32)[:n])
+def run(ctx, E, x, g, V, layout, chunk):
+    """(fused logits, fused index, logits of rrr_logits_rmsnorm, index of rrr_argmax_f32 on them)."""
+    Eh = orc.logits_chunk_build(E, K, V, chunk) if layout == rrr_hip.LOGITS_CHUNKED else E
+    Eb, xb, gb = ctx.to_device(Eh), ctx.to_device(x), ctx.to_device(g)
+    y1, y2, i1, i2 = ctx.alloc(V * 4), ctx.alloc(V * 4), ctx.alloc(4), ctx.alloc(4)
+    ctx.logits_rmsnorm_argmax(xb, gb, 1e-5, Eb, y1, K, V, i1, layout, chunk)
+    ctx.logits_rmsnorm(xb, gb, 1e-5, Eb, y2, K, V, layout, chunk)
+    ctx.argmax_f32(y2, V, i2)
+    out = (ctx.download(y1), int(ctx.download(i1, np.uint32, 1)[0]), ctx.download(y2),
+           int(ctx.download(i2, np.uint32, 1)[0]))
+    # again: the counters came back to zero
+    ctx.fill_u32(i1, 0xFFFFFFFF)
+    ctx.logits_rmsnorm_argmax(xb, gb, 1e-5, Eb, y1, K, V, i1, layout, chunk)
+    assert int(ctx.download(i1, np.uint32, 1)[0]) == out[1]
+    for b in (Eb, xb, gb, y1, y2, i1, i2):
+        b.free()
+    return out
+
+
+def check(ctx, E, x, g, V, layout, chunk, expect=None):
+    y, idx, y_ref, idx_ref = run(ctx, E, x, g, V, layout, chunk)
+    assert np.array_equal(y.view(np.uint32), y_ref.view(np.uint32))
+    assert idx == idx_ref == host_argmax(y_ref)
+    if expect is not None:
+        assert idx == expect
+    return y
+
+
+def inputs(V, seed):
+    E = synth.normal_f32(seed, V, V * K, 0.0, 0.02).reshape(V, K)
+    x = synth.normal_f32(seed, 1, K)
+    g = synth.normal_f32(seed, 2, K, 1.0, 0.1)
+    return E, x, g
+
+
+@pytest.mark.parametrize("V,chunk", [(20000, 8192), (65659, 8192), (1000, 256), (8195, 4096), (300, 8192)])
+def test_fused_argmax_matches(ctx, V, chunk):
+    E, x, g = inputs(V, 21)
+    check(ctx, E.reshape(-1), x, g, V, rrr_hip.LOGITS_CHUNKED, chunk)
+
+
+def test_fused_argmax_rows_layout(ctx):
+    E, x, g = inputs(5000, 22)
+    check(ctx, E.reshape(-1), x, g, 5000, rrr_hip.LOGITS_ROWS, 0)
+
+
+def test_fused_argmax_planted_ties_nan_inf(ctx):
+    V, chunk = 20000, 8192
+    E, x, g = inputs(V, 23)
+    normed = orc.rms_norm(x, g, 1e-5)
+    big = (0.01 * normed).astype(np.float32)      # a logit far above every random row's
+    # a tie across chunks and slabs: rows 17000 (chunk 2) and 300 (chunk 0)
+    E[17000] = big
+    E[300] = big
+    # a row whose logit is NaN (inf * mixed signs) never wins
+    E[50] = np.inf
+    check(ctx, E.reshape(-1), x, g, V, rrr_hip.LOGITS_CHUNKED, chunk, expect=300)
+    # a tie inside one slab (entries 9000 and 9003 of chunk 1), above the first
+    E[9003] = 2 * big
+    E[9000] = 2 * big
+    check(ctx, E.reshape(-1), x, g, V, rrr_hip.LOGITS_CHUNKED, chunk, expect=9000)
+    # +inf logits (one infinite weight where the normed input is positive):
+    # the first of them wins over every finite logit
+    k0 = int(np.flatnonzero(normed > 0)[0])
+    for r in (15000, 12345):
+        E[r] = 0.0
+        E[r, k0] = np.inf
+    y = check(ctx, E.reshape(-1), x, g, V, rrr_hip.LOGITS_CHUNKED, chunk, expect=12345)
+    assert np.isposinf(y[12345]) and np.isposinf(y[15000]) and np.isnan(y[50])
+
+
+def test_fused_argmax_graph_replay(ctx):
+    V, chunk = 20000, 8192
+    E, x, g = inputs(V, 24)
+    Eb = ctx.to_device(orc.logits_chunk_build(E.reshape(-1), K, V, chunk))
+    xb, gb = ctx.to_device(x), ctx.to_device(g)
+    y, i = ctx.alloc(V * 4), ctx.alloc(4)
+    ctx.logits_rmsnorm_argmax(xb, gb, 1e-5, Eb, y, K, V, i, rrr_hip.LOGITS_CHUNKED, chunk)
+    want_y, want_i = ctx.download(y), int(ctx.download(i, np.uint32, 1)[0])
+    ctx.graph_begin()
+    ctx.logits_rmsnorm_argmax(xb, gb, 1e-5, Eb, y, K, V, i, rrr_hip.LOGITS_CHUNKED, chunk)
+    gr = ctx.graph_end()
+    for _ in range(3):
+        ctx.fill_u32(y, 0)
+        ctx.fill_u32(i, 0xFFFFFFFF)
+        gr.launch()
+        ctx.sync()
+        assert int(ctx.download(i, np.uint32, 1)[0]) == want_i
+        assert np.array_equal(ctx.download(y).view(np.uint32), want_y.view(np.uint32))
+    gr.destroy()
+    for b in (Eb, xb, gb, y, i):
+        b.free()
