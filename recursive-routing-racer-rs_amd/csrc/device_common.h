@@ -209,17 +209,17 @@ __device__ __forceinline__ float lanes4_sum(float v)
 
 // Sum of the n <= NMAX values p[0], p[stride], ..., p[(n - 1) stride] (LDS)
 // in index order, every one requested before the first add (one LDS wait
-// instead of one per value); n >= 1.
-template <int NMAX>
+// instead of one per value), in T; n >= 1.
+template <int NMAX, class T = float>
 __device__ __forceinline__ float ordered_sum(const float *p, uint32_t n, uint32_t stride)
 {
     float q[NMAX];
 #pragma unroll
     for (uint32_t k = 0; k < NMAX; k++) q[k] = p[stride * min(k, n - 1)];
-    float v = q[0];
+    T v = q[0];
 #pragma unroll
-    for (uint32_t k = 1; k < NMAX; k++) v = k < n ? v + q[k] : v;
-    return v;
+    for (uint32_t k = 1; k < NMAX; k++) v = k < n ? v + (T)q[k] : v;
+    return (float)v;
 }
 
 // Deterministic full-wave sum: the xor butterfly over lane distances 32, 16,
