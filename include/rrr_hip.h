@@ -144,8 +144,7 @@ int rrr_dequant(rrr_ctx *ctx, uint32_t type, const rrr_buf *W, rrr_buf *out, uin
  * row up to M = 16; above 16 rows the K-quant rows run on the fp16 matrix
  * cores (Q4_K / Q5_K with K <= 3072 up to 32 rows, every K-quant shape with
  * N % 64 == 0, X and Y 16-byte aligned, beyond: X as f16 rows with a
- * power-of-two scale per row, zero-padded to 128 rows in the context
- * workspace) within 2e-3. */
+ * power-of-two scale per row, zero-padded in the context workspace) within 2e-3. */
 int rrr_gemv(rrr_ctx *ctx, const rrr_buf *X, const rrr_buf *W, uint32_t type, rrr_buf *Y,
              uint32_t K, uint32_t N, uint32_t M);
 
@@ -371,8 +370,9 @@ int rrr_logits_rmsnorm(rrr_ctx *ctx, const rrr_buf *x, const rrr_buf *gamma, flo
  * the final logits dispatches (phi4.rs:1049-1064) and the host argmax over
  * the mapped chunks (phi4.rs:1172-1183) in one call.  On the transposed-chunk
  * layout the argmax runs inside the logits launch (the last workgroup of each
- * 256-entry slab reduces the slab, the last slab reduces the slabs); the
- * logits are bit-identical to rrr_logits_rmsnorm's. */
+ * 256-entry slab reduces the slab, the last slab reduces the slabs), and on
+ * Q6_K rows the logits launch leaves each workgroup's candidate; the logits
+ * are bit-identical to rrr_logits_rmsnorm's. */
 int rrr_logits_rmsnorm_argmax(rrr_ctx *ctx, const rrr_buf *x, const rrr_buf *gamma, float eps,
                               const rrr_buf *E, rrr_buf *logits, uint32_t K, uint32_t V,
                               uint32_t layout, uint32_t chunk, rrr_buf *out_index);

@@ -536,8 +536,8 @@ __global__ __launch_bounds__(64 * WMAX) void skinny_kernel(GemvArgs a, uint32_t 
                     pp[(ti * MP + tt * TPT + (HILO ? 2 * kg + j : 4 * kg + j)) * 16] = tot[ti][tt][j];
         __syncthreads();
         // the W waves' partials in wave order, in 64 bits (a 12-long f32 chain
-        // was a third of the error: K = 8192, normal rows, Q4_K 1.35e-7 ->
-        // 1.20e-7 of the exact product's norm, Q6_K 1.33e-7 -> 1.20e-7; the
+        // was a fifth of the squared error: K = 8192, normal rows, Q4_K 1.36e-7 ->
+        // 1.23e-7 of the exact product's norm, Q6_K 1.33e-7 -> 1.20e-7; the
         // VALU kernel 1.23e-7 and 2.0e-7; no time)
         for (uint32_t i = t; i < T * MP * 16; i += 64 * W) {
             const uint32_t ti = i / (MP * 16), m = (i >> 4) % MP, c = i & 15, row = (tb0 + ti * GR) * 16 + c;
