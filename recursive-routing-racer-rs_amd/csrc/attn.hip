@@ -640,6 +640,10 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
 // P * 2^12 (P <= 8), undone exactly on the scores and at the end; the lo
 // parts then stay in f16's normal range, where they keep their precision.
 // The Q^T operands sit in LDS and are read per block.
+// Keys hidden from a token enter the products with P = 0, and 0 times a V that
+// is not finite is NaN: in the blocks with hidden keys (the last one of a wave at
+// most, in a form of its own, whose check runs under its MFMAs) such V are taken
+// out of V^T, and the tokens that see them get NaN at the end.
 constexpr uint32_t ATTM_LD = 36;   // f16 per V^T row in LDS (32 keys + pad; 72-byte rows)
 constexpr float ATTM_PS = 4096.0f;
 constexpr uint32_t ATTM_WAVES = 4, ATTM_OLD = ATT_HD + 4;   // waves; floats per merged output row (padded)
@@ -659,7 +663,8 @@ struct AttmLds {
     // the loop's V^T and Q^T share their bytes with the merge's outputs
     static constexpr size_t CW = (size_t)16 * (ATTM_WAVES + 1) * 4;             // merge: weights, scale
     static constexpr size_t LOOP = VT + Q, MAIN = LOOP > O ? LOOP : O;
-    static constexpr size_t BYTES = MAIN + ML + CW;
+    static constexpr size_t BAD = ATT_HD * 4;                                         // see `bad`
+    static constexpr size_t BYTES = MAIN + ML + CW + BAD;
 };
 
 template <bool F16OUT>
@@ -680,10 +685,13 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
     float *mml = (float *)(sm + LD::MAIN);                          // merge max / sum
     float *mcw = (float *)(sm + LD::MAIN + LD::ML);                 // merge weights and scale per token
     h8 *qop = (h8 *)(sm + LD::VT);                                  // Q^T operands [h][kk][hi, lo][lane]
+    uint32_t *bad = (uint32_t *)(sm + LD::MAIN + LD::ML + LD::CW);  // per dim the first cache row whose V was taken out
+    if (threadIdx.x < ATT_HD) bad[threadIdx.x] = ~0u;
     const uint32_t g = blockIdx.x, tb = blockIdx.y, l = threadIdx.x & 63, n = l & 15, grp = l >> 4;
     const uint32_t tok = tb * 16 + n, tq = min(tok, rows - 1), tpos = pos0 + tq;
     const uint32_t last = pos0 + min(tb * 16 + 15, rows - 1);      // the last cache row the block's tokens see
     const uint32_t nblk = last / 32 + 1;
+    const uint32_t nfull = (pos0 + tb * 16 + 1) / 32;              // blocks whose keys all tokens see
     const uint16_t *kbase = kc + (size_t)(g / heads_per_kv) * ATT_HD, *vbase = vc + (size_t)(g / heads_per_kv) * ATT_HD;
 
     // K and V of block blk (rows past `last` repeat it): the next block of
@@ -760,7 +768,7 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
 #pragma unroll
         for (int dt = 0; dt < 8; dt++) o[dt] = f4{0.f, 0.f, 0.f, 0.f};
     }
-    auto process = [&](uint32_t blk, const h8 (&ka)[2][4], const h8 (&vr)[2][4]) {
+    auto process = [&](uint32_t blk, const h8 (&ka)[2][4], const h8 (&vr)[2][4], auto hidden) {
         const uint32_t c0 = 32 * blk;
         // this wave's V^T (the wave's LDS operations run in order: the
         // previous block's reads come before these writes)
@@ -772,6 +780,14 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
                 *(h4 *)(vt + (8 * n + d) * ATTM_LD + 16 * half + 4 * grp) =
                     h4{vr[half][0][d], vr[half][1][d], vr[half][2][d], vr[half][3][d]};
         wave_lds_order();
+        uint64_t poison = 0;
+        if constexpr (hidden) {   // 0 stays 0 through these FMAs but for a V that is not finite
+            h8 z = {};
+#pragma unroll
+            for (int j = 0; j < 8; j++) z = __builtin_elementwise_fma(vr[j >> 2][j & 3], h8{}, z);
+            const u32x4 zb = __builtin_bit_cast(u32x4, z);
+            poison = __builtin_amdgcn_ballot_w64((zb.x | zb.y | zb.z | zb.w) != 0u);
+        }
         {
             h8 qh[4], ql[4];
 #pragma unroll
@@ -796,7 +812,7 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     sc[kt][r] *= qs;
-                    if (c0 + 16 * kt + 4 * grp + r > tpos) sc[kt][r] = -__builtin_inff();
+                    if (hidden && c0 + 16 * kt + 4 * grp + r > tpos) sc[kt][r] = -__builtin_inff();
                     bm = fmaxf(bm, sc[kt][r]);
                 }
             bm = lanes4_max(bm);
@@ -830,6 +846,18 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
             ps = lanes4_sum(ps);
             ls = fmaf(ls, cf, ps);
             m = mn;
+            if (hidden && __builtin_expect(poison != 0, 0)) {
+#pragma unroll 1
+                for (uint32_t i = 0; i < 64; i++) {
+                    const uint32_t dim = 8 * n + (i & 7), k = 16 * (i >> 5) + 4 * grp + ((i >> 3) & 3);
+                    _Float16 *e = vt + dim * ATTM_LD + k;
+                    if (!__builtin_isfinite((float)*e)) {
+                        atomicMin(bad + dim, c0 + k);
+                        *e = (_Float16)0.0f;
+                    }
+                }
+                wave_lds_order();
+            }
             // V^T operands of the 8 dim tiles read first, then the 8 P-hi
             // MFMAs and the 8 P-lo MFMAs (each accumulator takes hi then lo)
             h8 av[8];
@@ -846,17 +874,24 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
         }
     };
     {   // two register sets
+        const std::bool_constant<false> seen;
+        const std::bool_constant<true> hidden;
         h8 kaB[2][4], vrB[2][4];
         uint32_t blk = wv;
-        while (blk < nblk) {
+        while (blk < nfull) {
             load_blk(min(blk + ATTM_WAVES, nblk - 1), kaB, vrB);   // past the last block: a repeat, unused
-            process(blk, kaA, vrA);
+            process(blk, kaA, vrA, seen);
             blk += ATTM_WAVES;
-            if (blk >= nblk) break;
+            if (blk >= nfull) {
+                if (blk < nblk) process(blk, kaB, vrB, hidden);
+                blk = nblk;
+                break;
+            }
             load_blk(min(blk + ATTM_WAVES, nblk - 1), kaA, vrA);
-            process(blk, kaB, vrB);
+            process(blk, kaB, vrB, seen);
             blk += ATTM_WAVES;
         }
+        if (blk < nblk) process(blk, kaA, vrA, hidden);   // nfull + 2 >= nblk: a wave's last
     }
     // merge the waves: wave w's output rows (token, dims) and its max / sum
     // per token; a wave without blocks holds max -inf, sum 0
@@ -908,7 +943,7 @@ __global__ __launch_bounds__(64 * ATTM_WAVES) void attn_prefill_mfma_kernel(cons
             const float sc = cw[ATTM_WAVES];
             f4 v;
 #pragma unroll
-            for (int e = 0; e < 4; e++) v[e] = O[e] * sc;
+            for (int e = 0; e < 4; e++) v[e] = bad[d + e] <= pos0 + tk ? __builtin_nanf("") : O[e] * sc;
             if constexpr (F16OUT) {
                 asm volatile("" : "+v"(v));   // the f32 results, then their rounding (no mixed-precision fold)
                 *(h4 *)((_Float16 *)out + oi) = h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};

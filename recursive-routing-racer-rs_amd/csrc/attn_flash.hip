@@ -21,6 +21,10 @@
 //                   the same order: keys 16 m + 4 (l / 32) + {0..3, 8..11}, two
 //                   transposing LDS reads (ds_read_b64_tr_b16: 16 lanes address
 //                   4 keys x 16 dims, lane i gets dim i of the 4 keys).
+// A wave stops at the tile with its last row's last key and then only loads for
+// the others.  Hidden keys in the tiles before enter the product with P = 0, and
+// 0 times a V that is not finite would be NaN: such V are taken out of the
+// operand, and the rows that do see them get their NaN at the end.
 // The hi + lo scalings are those of the short form in attn.hip: Q by a power of
 // two per row that puts its largest component in [2^13, 2^14), P (<= 8) by 2^12.
 //
@@ -47,6 +51,7 @@ struct AfGeom {
     static constexpr uint32_t MERGE = (8 - RG) * 64 * (64 + 2) * 4;   // the other waves' O, max, sum
     static constexpr uint32_t NS = KQ == 2 ? 3 : 2;                   // places of a K and V tile in LDS
     static constexpr uint32_t LDS = 2 * NS * TILE > MERGE ? 2 * NS * TILE : MERGE;
+    static constexpr uint32_t BYTES = LDS + (ATT_HD + 1) * 4;         // and the first rows with a V that is not finite
 };
 
 __device__ __forceinline__ f16x4a lds_tr4(const uint8_t *p)
@@ -91,6 +96,8 @@ __global__ __launch_bounds__(512) void attn_flash_kernel(const float *__restrict
     const uint32_t wlo = pos0 + min(R0, total - 1) / hpk;                       // the wave's first row's last key
     const uint32_t last = pos0 + min(32 * RG * (b + 1) - 1, total - 1) / hpk;   // the workgroup's last key
     const uint32_t tiles = last / TK + 1, kv_stride = n_kv * ATT_HD;
+    const uint32_t whi = pos0 + min(R0 + 31, total - 1) / hpk;                  // the wave's last key
+    const uint32_t mine = whi >= 32 * kq ? (whi - 32 * kq) / TK + 1 : 0u;       // the wave's tiles with a key of its rows
 
     // K and V tiles: load i of a wave covers cache rows 4 (wave + 8 i) .. + 3 of
     // the tile, lane l row l / 16 and the 16-byte chunk whose place is l % 16:
@@ -169,8 +176,11 @@ __global__ __launch_bounds__(512) void attn_flash_kernel(const float *__restrict
             v[x] = lds_tr4(af_lds + (va ^ (64u * dt ^ 32u * x)) + 256 * (16 * k2 + 8 * x));
         return __builtin_shufflevector(v[0], v[1], 0, 1, 2, 3, 4, 5, 6, 7);
     };
+    // per dim the first cache row whose V was taken out, then whether any was
+    uint32_t *bad = (uint32_t *)(af_lds + G::LDS);
+    if (threadIdx.x < ATT_HD + 1) bad[threadIdx.x] = threadIdx.x < ATT_HD ? ~0u : 0u;
     uint32_t st = 0;   // place of tile t
-    for (uint32_t t = 0; t < tiles; t++) {
+    for (uint32_t t = 0; t < mine; t++) {
         // tile t landed in every wave, and every wave is done with tile t - 1
         wait_vm<(G::NS - 2) * 2 * KQ>();
         barrier_lds();
@@ -194,9 +204,15 @@ __global__ __launch_bounds__(512) void attn_flash_kernel(const float *__restrict
             __builtin_amdgcn_sched_barrier(0);
         }
         float bm = -__builtin_inff();
+        bool poison = false;   // a V that is not finite, in a tile with hidden keys
 #pragma unroll
         for (int r = 0; r < 16; r++) s[r] = s[r] + s2[r];
         if (c0 + 31 > wlo) {   // the tile holds keys past some of the wave's rows
+            f16x8a z = {};
+#pragma unroll
+            for (int i = 0; i < 8; i++) z = __builtin_elementwise_fma(av[i >> 2][i & 3], f16x8a{}, z);
+            const u32x4 zb = __builtin_bit_cast(u32x4, z);
+            poison = __builtin_amdgcn_ballot_w64((zb.x | zb.y | zb.z | zb.w) != 0u) != 0;
 #pragma unroll
             for (int r = 0; r < 16; r++)
                 if (c0 + 8 * (r >> 2) + 4 * hb + (r & 3) > tpos) s[r] = -__builtin_inff();
@@ -238,6 +254,21 @@ __global__ __launch_bounds__(512) void attn_flash_kernel(const float *__restrict
             __builtin_amdgcn_sched_barrier(0);
         }
         ls += lt;
+        if (__builtin_expect(poison, 0)) {
+#pragma unroll
+            for (int k2 = 0; k2 < 2; k2++)
+#pragma unroll
+                for (int dt = 0; dt < 4; dt++) {
+#pragma unroll
+                    for (int i = 0; i < 8; i++)
+                        if (!__builtin_isfinite((float)av[k2][dt][i])) {
+                            atomicMin(bad + 32 * dt + (lane & 31), c0 + 16 * k2 + 8 * (i >> 2) + 4 * hb + (i & 3));
+                            bad[ATT_HD] = 1;
+                            av[k2][dt][i] = (_Float16)0.0f;
+                        }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+        }
 #pragma unroll
         for (int k2 = 0; k2 < 2; k2++) {
 #pragma unroll
@@ -245,6 +276,14 @@ __global__ __launch_bounds__(512) void attn_flash_kernel(const float *__restrict
 #pragma unroll
             for (int dt = 0; dt < 4; dt++) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[k2][dt], pl[k2], o[dt], 0, 0, 0);
         }
+        st = st + 1 == G::NS ? 0 : st + 1;
+    }
+    for (uint32_t t = mine; t < tiles; t++) {   // the other waves' tiles
+        wait_vm<(G::NS - 2) * 2 * KQ>();
+        barrier_lds();
+        const uint32_t sp = st == 0 ? G::NS - 1 : st - 1;
+#pragma unroll
+        for (int i = 0; i < 2 * KQ; i++) load_part(t + G::NS - 1, sp, i);
         st = st + 1 == G::NS ? 0 : st + 1;
     }
     wait_vm<0>();   // the repeated tile's loads, before the LDS is used again
@@ -280,6 +319,7 @@ __global__ __launch_bounds__(512) void attn_flash_kernel(const float *__restrict
     }
     // registers 4 q .. 4 q + 3 are dims 8 q + 4 hb ..; lanes l and l ^ 32 swap
     // so that one holds 8 dims of quad q, the other of quad q + 1
+    const uint32_t any_bad = bad[ATT_HD];
     const float inv = 1.0f / ls;
     const size_t oi = ((size_t)tok * n_kv * hpk + head) * ATT_HD;
 #pragma unroll
@@ -295,7 +335,13 @@ __global__ __launch_bounds__(512) void attn_flash_kernel(const float *__restrict
                 v[4 + i] = u2f(w[1]);
             }
             if (R >= total) continue;
-            const size_t d = oi + 32 * dt + 8 * (q + hb);
+            const uint32_t dim = 32 * dt + 8 * (q + hb);
+            if (__builtin_expect(any_bad != 0, 0)) {
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+                    if (bad[dim + i] <= tpos) v[i] = __builtin_nanf("");
+            }
+            const size_t d = oi + dim;
             if constexpr (F16OUT) {
                 f16x8a h;
 #pragma unroll
@@ -318,10 +364,10 @@ static hipError_t go_flash(const float *qkv, uint32_t row_stride, uint32_t rows,
     using G = AfGeom<KQ>;
     const uint32_t blocks = (rows * hpk + 32 * G::RG - 1) / (32 * G::RG);
     if (out_f16)
-        hipLaunchKernelGGL((attn_flash_kernel<KQ, true>), dim3(blocks * n_kv), dim3(512), G::LDS, s, qkv, row_stride, kc,
+        hipLaunchKernelGGL((attn_flash_kernel<KQ, true>), dim3(blocks * n_kv), dim3(512), G::BYTES, s, qkv, row_stride, kc,
                            vc, out, rows, pos0, n_kv, hpk, blocks, qscale);
     else
-        hipLaunchKernelGGL((attn_flash_kernel<KQ, false>), dim3(blocks * n_kv), dim3(512), G::LDS, s, qkv, row_stride, kc,
+        hipLaunchKernelGGL((attn_flash_kernel<KQ, false>), dim3(blocks * n_kv), dim3(512), G::BYTES, s, qkv, row_stride, kc,
                            vc, out, rows, pos0, n_kv, hpk, blocks, qscale);
     return hipGetLastError();
 }
