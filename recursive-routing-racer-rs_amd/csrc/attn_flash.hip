@@ -245,8 +245,10 @@ __global__ __launch_bounds__(512) void attn_flash_kernel(const float *__restrict
             const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], qs, off));
             const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r + 1], qs, off));
             lt += p0 + p1;
-            const f16x2a hi = __builtin_bit_cast(f16x2a, __builtin_amdgcn_cvt_pkrtz(p0, p1));
-            const f16x2a lo = __builtin_bit_cast(f16x2a, __builtin_amdgcn_cvt_pkrtz(p0 - (float)hi[0], p1 - (float)hi[1]));
+            // both halves to nearest: what they lose has no sign (cut off, every
+            // output came 7e-8 of its size short)
+            const f16x2a hi = {(_Float16)p0, (_Float16)p1};
+            const f16x2a lo = {(_Float16)(p0 - (float)hi[0]), (_Float16)(p1 - (float)hi[1])};
             pb[r >> 3][r & 7] = hi[0];
             pb[r >> 3][(r & 7) + 1] = hi[1];
             pl[r >> 3][r & 7] = lo[0];
