@@ -29,11 +29,17 @@
 // two per row that puts its largest component in [2^13, 2^14), P (<= 8) by 2^12.
 //
 // Bound: a wave's chain through a tile (LDS reads, 16 MFMAs, the softmax, 16
-// MFMAs: 1.65 us, of which 0.9 us MFMA for the SIMD's two waves).  2,000 rows
-// of 8 x 3 heads 76 us (156 with a wave to 16 tokens and keys read by every
-// wave), 1,000 rows 33 (57), 512 rows behind 256 22 (31).  Measured and not
-// kept: the next tile's scores between the exponentials (registers spill: 81
-// us), the upper waves' outputs one step late (75 to 85 us).
+// MFMAs: 1.65 us, of which 0.9 us MFMA for the SIMD's two waves).  In prompts,
+// 2,000 rows of 8 x 3 heads 76 us (156 with a wave to 16 tokens and keys read by
+// every wave), 1,000 rows 33 (57), 512 rows behind 256 22 (31); eight in a row
+// from one graph 62, 30 and 20.  Measured and not kept: the next tile's scores
+// between the exponentials (registers spill: 81 us), the upper waves' outputs one
+// step late (75 to 85 us).
+// Precision, to 64 bits, against the per-head form on the same rows: scores of
+// standard deviation 1.5 2.4e-7 to 2.9e-7 (3.2e-7 to 3.9e-7), 6 4.7e-7 to
+// 5.2e-7 (6.7e-7 to 7.2e-7); near 0, where the f32 sums are all of it, 1.0e-7 to
+// 1.4e-7 on tiles of 128 keys (1.1e-7 to 1.5e-7) and 1.25e-7 to 1.35e-7 on tiles
+// of 64, whose waves add up twice the keys (1.2e-7).
 #include "device_common.h"
 #include "internal.h"
 
@@ -187,26 +193,27 @@ __global__ __launch_bounds__(512) void attn_flash_kernel(const float *__restrict
         const uint32_t c0 = t * TK + 32 * kq, sp = st == 0 ? G::NS - 1 : st - 1;   // sp: place of t - 1 and t + NS - 1
         uint32_t ka = kaddr + st * 2 * G::TILE, va = vaddr + st * 2 * G::TILE;
         asm volatile("" : "+v"(ka), "+v"(va));   // the fragments' addresses are made where they are used
-        f32x16 s, s2;
+        f32x16 s;
 #pragma unroll
-        for (int r = 0; r < 16; r++) s[r] = s2[r] = 0.0f;
+        for (int r = 0; r < 16; r++) s[r] = 0.0f;
         f16x8a kf[8], av[2][4];
 #pragma unroll
         for (int kk = 0; kk < 8; kk++) kf[kk] = kfrag(ka, kk);
         __builtin_amdgcn_sched_barrier(0);
         // all V^T reads here, between the MFMAs: ahead of the next DMA, for
-        // which the compiler would make a transposing read wait
+        // which the compiler would make a transposing read wait.  The lo products
+        // first, in the same sums: they round at their own size, and there is no
+        // second sum to add
 #pragma unroll
         for (int kk = 0; kk < 8; kk++) {
-            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[kk], qh[kk], s, 0, 0, 0);
-            s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[kk], ql[kk], s2, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[kk], ql[kk], s, 0, 0, 0);
             av[kk >> 2][kk & 3] = vfrag(va, kk >> 2, kk & 3);
             __builtin_amdgcn_sched_barrier(0);
         }
+#pragma unroll
+        for (int kk = 0; kk < 8; kk++) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[kk], qh[kk], s, 0, 0, 0);
         float bm = -__builtin_inff();
         bool poison = false;   // a V that is not finite, in a tile with hidden keys
-#pragma unroll
-        for (int r = 0; r < 16; r++) s[r] = s[r] + s2[r];
         if (c0 + 31 > wlo) {   // the tile holds keys past some of the wave's rows
             f16x8a z = {};
 #pragma unroll
@@ -234,7 +241,7 @@ __global__ __launch_bounds__(512) void attn_flash_kernel(const float *__restrict
                 for (int r = 0; r < 16; r++) o[dt][r] *= cf;
         }
         m = mn;
-        const float off = 12.0f - (mn == -__builtin_inff() ? 0.0f : mn);
+        const float off = mn == -__builtin_inff() ? 0.0f : -mn;
         f16x8a pb[2], pl[2];
         float lt = 0.0f;
         // a tile's loads between the exponentials (in a row they hold the wave
@@ -242,8 +249,10 @@ __global__ __launch_bounds__(512) void attn_flash_kernel(const float *__restrict
 #pragma unroll
         for (int r = 0; r < 16; r += 2) {
             if (r / 2 < 2 * KQ) load_part(t + G::NS - 1, sp, r / 2);
-            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], qs, off));
-            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r + 1], qs, off));
+            // 2^12 by a product: in the exponent it would cost its argument, near 0
+            // for the weights that count, up to four bits
+            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], qs, off)) * 4096.0f;
+            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r + 1], qs, off)) * 4096.0f;
             lt += p0 + p1;
             // both halves to nearest: what they lose has no sign (cut off, every
             // output came 7e-8 of its size short)

@@ -43,3 +43,24 @@ def test_weights_lose_nothing_on_average(ctx, kv, hpk, M, pos):
     qkv, K, V = inputs(kv, hpk, M, pos, 1.5)
     V[:] = 1.0
     assert abs(attend(ctx, qkv, K, V, kv, hpk, pos, M).mean() - 1.0) < 2.0 ** -25
+
+
+@pytest.mark.parametrize("kv,hpk,M,pos", SHAPES)
+def test_no_further_off_than_the_per_head_form(ctx, kv, hpk, M, pos):
+    """Small scores: weights near 1, whose exponents have an argument near 0.  The forms differ in the order of
+    their sums only: to 64 bits both are about 1.3e-7 off.  The longer sums of the shared tiles (twice the keys a
+    wave) may cost a factor of up to sqrt(2) where the sums are all of the error; with 2^12 in the exponent's
+    argument the factor was 2."""
+    qkv, K, V = inputs(kv, hpk, M, pos, 0.3)
+    tiles, heads = attend(ctx, qkv, K, V, kv, hpk, pos, M), attend(ctx, qkv, K, V, kv, hpk, pos, 64)
+    n = pos + M
+    q, k, v = (a.astype(np.float64) for a in (qkv[:, :kv * hpk * 128].reshape(M, kv * hpk, 128),
+                                              K.reshape(n, kv, 128), V.reshape(n, kv, 128)))
+    seen = np.arange(n)[None] <= pos + np.arange(M)[:, None]
+    err = {"tiles": 0.0, "heads": 0.0}
+    for h in range(0, kv * hpk, 5):
+        p = np.where(seen, np.exp(q[:, h] @ k[:, h // hpk].T / np.sqrt(128.0)), 0.0)
+        ref = (p / p.sum(1, keepdims=True)) @ v[:, h // hpk]
+        err["tiles"] += ((tiles[:, h] - ref) ** 2).sum()
+        err["heads"] += ((heads[:, h] - ref) ** 2).sum()
+    assert err["tiles"] <= 2.0 * err["heads"], err
