@@ -4,18 +4,27 @@
 // row-major).
 //
 // Exact weights.  For super-block b of row n,
-//     sum_k x_k w_k = d * sum_s sum_{k in s} (sc_s q_k) x_k - dmin * sum_s mn_s X_s
-// (phi4.rs:481-542, w = d*sc*q - dmin*mn), X_s the sum of x over sub-block s.
-// sc_s q_k <= 63 * 31 = 1953 < 2^11 is an integer, exact in fp16: the MFMA B
-// operand carries it, the 8 sub-blocks of a block accumulate in the MFMA's f32
-// accumulator, and d, dmin are applied once per block.  The min term is a
-// second, small MFMA (16x16x16) of the sub-block sums X_s against mn_s.
+//     sum_k x_k w_k = d * sum_s sum_{k in s} sc_s (q_k - c) x_k
+//                     + sum_s (c d sc_s - dmin mn_s) X_s
+// (phi4.rs:481-542, w = d*sc*q - dmin*mn), X_s the sum of x over sub-block s and c
+// the middle of the quants (8 or 16).  sc_s (q_k - c) is an integer of at most
+// 1008, exact in fp16: the MFMA B operand carries it, the 8 sub-blocks of a block
+// accumulate in the MFMA's f32 accumulator, and d, dmin are applied once per block.
+// The sums' terms are small MFMAs (16x16x16) of the X_s against sc_s and mn_s.
+// With c = 0 the f32 sums are those of products of one sign, about twice as large
+// as what they come to, and 4 times as far from it where x has a mean (M > 16, of
+// f16 activations, has c = 0: sc_s q_k <= 1953 < 2^11).
+// Error to 64 bits, M <= 16, K = 8192, weights of mean zero (with c = 0; the VALU
+// kernel's, f32 throughout): even rows Q4_K 1.1e-7 (2.5e-7; 1.9e-7), Q5_K 1.2e-7
+// (2.6e-7; 2.0e-7), Q6_K 1.2e-7 (VALU 2.0e-7); log-normal rows 1.3e-7 to 1.6e-7
+// (2.6e-7 to 3.0e-7; 1.8e-7 to 2.3e-7); rows with a mean 1.2e-7 to 1.7e-7
+// (1.8e-6; 4.1e-7 to 4.3e-7).
 //
 // Activations.  A wave's K slice (one super-block) of token m is scaled by
 // 2^-E (E from the slice maximum, so the values lie below 2^14) and split
-// x = hi + lo, hi = fp16(x), lo = fp16(x - hi), relative error 2^-22 of the
-// slice maximum.  M <= 16: A rows 2m+h (h = 0 hi, 1 lo), 8 tokens per 16-row A
-// tile (the GEMV bar, 1e-4).  16 < M <= 32: A rows are 16 tokens of hi only
+// x = hi + lo, hi = fp16(x), lo = fp16(x - hi), off by at most 2^-23 of x or 2^-39
+// of the slice maximum.  M <= 16: A rows 2m+h (h = 0 hi, 1 lo), 8 tokens per 16-row
+// A tile (the GEMV bar, 1e-4).  16 < M <= 32: A rows are 16 tokens of hi only
 // (error 2^-12, the MFMA bar 2e-3).  The X_s are scaled by 2^-(E+5)
 // (|X_s| <= 32 max) and split the same way; d and dmin take the 2^E back.
 //
@@ -27,7 +36,7 @@
 // (skinny_encode_kernel) builds them once per call into the workspace, in the
 // lane order of the MFMA:
 //   av   [TOK][B][8][64] f16x8  lane's 8 values of sub-block s
-//   amin [TOK][B][64]    f16x4  lane's 4 sub-block sums (min-term A operand)
+//   amin [TOK][B][64]    f16x4  lane's 4 sub-block sums (A operand of their terms)
 //   pe   [TOK][B][16]    f32    2^E of the A tile's token r (8 or 16 of them)
 // (B = K/256 columns, TOK A tiles), 8,768 bytes per (tile, column).  Every
 // workgroup of the main kernel then loads its operands with 16-byte loads
@@ -82,9 +91,11 @@ constexpr uint32_t SK_OOB = 0x80000000u;
 __device__ __forceinline__ f16x2s sk_bits(uint32_t v) { return __builtin_bit_cast(f16x2s, v); }
 __device__ __forceinline__ uint32_t sk_u32(f16x2s v) { return __builtin_bit_cast(uint32_t, v); }
 
-// Four quant values (bytes < 64 of v) times the scale as exact fp16:
-// v_perm places byte q under the exponent of 1024 (f16 0x64qq = 1024 + q),
-// and fma(1024 + q, sc, -1024 sc) = sc * q, exact (< 2^11).
+// Four quant values times the scale as exact fp16: v_perm places the bytes of v under
+// the exponent of 1024 (f16 0x64vv = 1024 + v).  Plain, the bytes are q and
+// fma(1024 + q, sc, -1024 sc) = sc q < 2^11; less their middle c, they are 64 q / c
+// and fma(1024 + 64 q / c, sc c / 64, -(1024 + 64) sc c / 64) = sc (q - c), where
+// 17 sc has 11 bits and |sc (q - c)| <= 1008.
 __device__ __forceinline__ void sk_scale4(uint32_t v, f16x2s sc2, f16x2s nb2, uint32_t &o01, uint32_t &o23)
 {
     o01 = sk_u32(__builtin_elementwise_fma(sk_bits(__builtin_amdgcn_perm(0x64646464u, v, 0x04010400u)), sc2, nb2));
@@ -96,6 +107,7 @@ __device__ __forceinline__ void sk_scale4(uint32_t v, f16x2s sc2, f16x2s nb2, ui
 struct SkQ4K {
     static constexpr uint32_t BS = 144, LROW = 144;   // bytes of a block, and of its row in LDS
     static constexpr bool MINS = true;                // a min term (d*sc*q - dmin*mn)
+    static constexpr uint32_t MID = 8;                // the middle of the quants
     struct Raw { u32x4 hdr; u32x2 qs[4]; };
     __device__ static void load(Raw &r, const uint8_t *L, uint32_t o, uint32_t kg, uint32_t)
     {
@@ -103,11 +115,18 @@ struct SkQ4K {
 #pragma unroll
         for (int p = 0; p < 4; p++) r.qs[p] = *(const u32x2 *)(L + o + 16 + 32 * p + 8 * kg);
     }
-    // quant values of sub-block s at the lane's 8 positions, one per byte
+    // quant values of sub-block s at the lane's 8 positions, one per byte (C: times 8)
+    template <bool C>
     __device__ static void quants(const Raw &r, int s, uint32_t &v0, uint32_t &v1)
     {
-        v0 = (r.qs[s >> 1].x >> (4 * (s & 1))) & 0x0F0F0F0Fu;
-        v1 = (r.qs[s >> 1].y >> (4 * (s & 1))) & 0x0F0F0F0Fu;
+        const u32x2 q = r.qs[s >> 1];
+        if constexpr (C) {
+            v0 = (s & 1 ? q.x >> 1 : q.x << 3) & 0x78787878u;
+            v1 = (s & 1 ? q.y >> 1 : q.y << 3) & 0x78787878u;
+        } else {
+            v0 = (q.x >> (4 * (s & 1))) & 0x0F0F0F0Fu;
+            v1 = (q.y >> (4 * (s & 1))) & 0x0F0F0F0Fu;
+        }
     }
 };
 
@@ -115,6 +134,7 @@ struct SkQ4K {
 struct SkQ5K {
     static constexpr uint32_t BS = 176, LROW = 176;
     static constexpr bool MINS = true;
+    static constexpr uint32_t MID = 16;
     struct Raw { u32x4 hdr; u32x2 qh; u32x2 qs[4]; };
     __device__ static void load(Raw &r, const uint8_t *L, uint32_t o, uint32_t kg, uint32_t)
     {
@@ -123,10 +143,17 @@ struct SkQ5K {
 #pragma unroll
         for (int p = 0; p < 4; p++) r.qs[p] = *(const u32x2 *)(L + o + 48 + 32 * p + 8 * kg);
     }
+    template <bool C>   // C: times 4
     __device__ static void quants(const Raw &r, int s, uint32_t &v0, uint32_t &v1)
     {
-        v0 = ((r.qs[s >> 1].x >> (4 * (s & 1))) & 0x0F0F0F0Fu) | (((r.qh.x >> s) & 0x01010101u) << 4);
-        v1 = ((r.qs[s >> 1].y >> (4 * (s & 1))) & 0x0F0F0F0Fu) | (((r.qh.y >> s) & 0x01010101u) << 4);
+        const u32x2 q = r.qs[s >> 1];
+        if constexpr (C) {
+            v0 = ((s & 1 ? q.x >> 2 : q.x << 2) & 0x3C3C3C3Cu) | ((s < 7 ? r.qh.x << (6 - s) : r.qh.x >> 1) & 0x40404040u);
+            v1 = ((s & 1 ? q.y >> 2 : q.y << 2) & 0x3C3C3C3Cu) | ((s < 7 ? r.qh.y << (6 - s) : r.qh.y >> 1) & 0x40404040u);
+        } else {
+            v0 = ((q.x >> (4 * (s & 1))) & 0x0F0F0F0Fu) | (((r.qh.x >> s) & 0x01010101u) << 4);
+            v1 = ((q.y >> (4 * (s & 1))) & 0x0F0F0F0Fu) | (((r.qh.y >> s) & 0x01010101u) << 4);
+        }
     }
 };
 
@@ -160,6 +187,7 @@ struct SkQ6K {
         r.sc[3] = __builtin_amdgcn_alignbyte(e, c.w, odd);
         r.d = e >> (8 * odd);
     }
+    template <bool>
     __device__ static void quants(const Raw &r, int s, uint32_t &v0, uint32_t &v1)
     {
         const int g = s >> 2, q = s & 3;
@@ -426,18 +454,25 @@ __global__ __launch_bounds__(64 * WMAX) void skinny_kernel(GemvArgs a, uint32_t 
             const float d = h2f(raw.hdr.x), dmin = h2f(raw.hdr.x >> 16);
             uint32_t scb[2], mnb[2];
             scale_min_bytes_k4(raw.hdr.y, raw.hdr.z, raw.hdr.w, scb, mnb);
-            // min term B operand: mn of sub-blocks 4 kg .. 4 kg + 3 (k-groups 2, 3 padding)
-            const uint32_t mk = kg == 0 ? mnb[0] : mnb[1];
-            const f16x2s m01 = sk_bits(__builtin_amdgcn_perm(0x64646464u, mk, 0x04010400u)) - k1024;
-            const f16x2s m23 = sk_bits(__builtin_amdgcn_perm(0x64646464u, mk, 0x04030402u)) - k1024;
-            const f16x4s bmin = kg < 2 ? f16x4s{m01[0], m01[1], m23[0], m23[1]} : f16x4s{(_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f};
+            // B operands of the sub-block sums: sc and mn of sub-blocks 4 kg .. 4 kg + 3
+            // (k-groups 2, 3 padding, whose A is 0)
+            auto bytes4 = [&](uint32_t v) {
+                const f16x2s a = sk_bits(__builtin_amdgcn_perm(0x64646464u, v, 0x04010400u)) - k1024;
+                const f16x2s b = sk_bits(__builtin_amdgcn_perm(0x64646464u, v, 0x04030402u)) - k1024;
+                return f16x4s{a[0], a[1], b[0], b[1]};
+            };
+            const f16x4s bsc = bytes4(kg == 0 ? scb[0] : scb[1]), bmin = bytes4(kg == 0 ? mnb[0] : mnb[1]);
 #pragma unroll
             for (int s = 0; s < 8; s++) {
-                // {sc_s, sc_s} exactly: byte s under the exponent of 1024, minus 1024
-                const f16x2s sc2 = sk_bits(__builtin_amdgcn_perm(0x64646464u, scb[s >> 2], 0x04000400u + 0x00010001u * (s & 3))) - k1024;
-                const f16x2s nb2 = sc2 * -k1024;
+                // {sc_s, sc_s}, for centred quants times MID / 64, exactly: byte s under the
+                // exponent of 1024 (16 MID), less that
+                constexpr uint32_t base = HILO ? 16 * Q::MID : 1024, ex = base == 128 ? 0x58585858u : base == 256 ? 0x5C5C5C5Cu : 0x64646464u;
+                const f16x2s sc2 = sk_bits(__builtin_amdgcn_perm(ex, scb[s >> 2], 0x04000400u + 0x00010001u * (s & 3))) -
+                                   f16x2s{(_Float16)base, (_Float16)base};
+                constexpr float off = HILO ? -1088.0f : -1024.0f;
+                const f16x2s nb2 = sc2 * f16x2s{(_Float16)off, (_Float16)off};
                 uint32_t v0, v1, b[4];
-                Q::quants(raw, s, v0, v1);
+                Q::template quants<HILO>(raw, s, v0, v1);
                 sk_scale4(v0, sc2, nb2, b[0], b[1]);
                 sk_scale4(v1, sc2, nb2, b[2], b[3]);
                 const f16x8s bv = __builtin_bit_cast(f16x8s, u32x4{b[0], b[1], b[2], b[3]});
@@ -446,15 +481,30 @@ __global__ __launch_bounds__(64 * WMAX) void skinny_kernel(GemvArgs a, uint32_t 
                 // one sub-block's B operand live at a time
                 if constexpr (TOK > 1) __builtin_amdgcn_sched_barrier(0);
             }
-            // the row partials: d * 2^E * S - dmin * 2^(E+5) * S_min
+            // the row partials
+            const float ds = (32.0f * Q::MID) * d, dm = 32.0f * dmin;
+            const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int tt = 0; tt < TOK; tt++) {
-                const f32x4 accm = __builtin_amdgcn_mfma_f32_16x16x16f16(x.amin[tt], bmin, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                const f32x4 sm = __builtin_amdgcn_mfma_f32_16x16x16f16(x.amin[tt], bmin, zero, 0, 0, 0);
+                if constexpr (HILO) {
+                    // the two terms of the X_s nearly cancel where these are large: the
+                    // difference of the hi parts is taken exactly (the product's rounding
+                    // comes back), then the lo parts join
+                    const f32x4 ss = __builtin_amdgcn_mfma_f32_16x16x16f16(x.amin[tt], bsc, zero, 0, 0, 0);
 #pragma unroll
-                for (int j = 0; j < DPT; j++) {
-                    const float sv = HILO ? acc[tt][2 * j] + acc[tt][2 * j + 1] : acc[tt][j];
-                    const float sm = HILO ? accm[2 * j] + accm[2 * j + 1] : accm[j];
-                    tot[ti][tt][j] = fmaf(x.pe[tt][j], fmaf(d, sv, -(32.0f * dmin) * sm), tot[ti][tt][j]);
+                    for (int j = 0; j < DPT; j++) {
+                        const int h = 2 * j;
+                        const float p = dm * sm[h];
+                        float v = fmaf(ds, ss[h], -p) - fmaf(dm, sm[h], -p);
+                        v = fmaf(-dm, sm[h + 1], fmaf(ds, ss[h + 1], v));
+                        v = fmaf(d, acc[tt][h], fmaf(d, acc[tt][h + 1], v));
+                        tot[ti][tt][j] = fmaf(x.pe[tt][j], v, tot[ti][tt][j]);
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < DPT; j++)
+                        tot[ti][tt][j] = fmaf(x.pe[tt][j], fmaf(d, acc[tt][j], -dm * sm[j]), tot[ti][tt][j]);
                 }
             }
         } else {
@@ -466,7 +516,7 @@ __global__ __launch_bounds__(64 * WMAX) void skinny_kernel(GemvArgs a, uint32_t 
                 const f16x2s sc2 = sk_bits(__builtin_amdgcn_perm(0x64646464u, raw.sc[s >> 1] ^ 0x80808080u, sel + 0x00020002u * (s & 1))) -
                                    f16x2s{(_Float16)1152.0f, (_Float16)1152.0f};
                 uint32_t v0, v1, h0[2], h1[2], l0[2], l1[2];
-                Q::quants(raw, s, v0, v1);
+                Q::template quants<HILO>(raw, s, v0, v1);
                 sk_scale4_q6(v0, sc2, h0, l0);
                 sk_scale4_q6(v1, sc2, h1, l1);
                 const f16x8s bh = __builtin_bit_cast(f16x8s, u32x4{h0[0], h0[1], h1[0], h1[1]});
@@ -535,10 +585,8 @@ __global__ __launch_bounds__(64 * WMAX) void skinny_kernel(GemvArgs a, uint32_t 
                 for (int j = 0; j < DPT; j++)
                     pp[(ti * MP + tt * TPT + (HILO ? 2 * kg + j : 4 * kg + j)) * 16] = tot[ti][tt][j];
         __syncthreads();
-        // the W waves' partials in wave order, in 64 bits (a 12-long f32 chain
-        // was a fifth of the squared error: K = 8192, normal rows, Q4_K 1.36e-7 ->
-        // 1.23e-7 of the exact product's norm, Q6_K 1.33e-7 -> 1.20e-7; the
-        // VALU kernel 1.23e-7 and 2.0e-7; no time)
+        // the W waves' partials in wave order, in 64 bits (a 12-long f32 chain was a
+        // tenth of the error; no time)
         for (uint32_t i = t; i < T * MP * 16; i += 64 * W) {
             const uint32_t ti = i / (MP * 16), m = (i >> 4) % MP, c = i & 15, row = (tb0 + ti * GR) * 16 + c;
             if (m < M && row < N) {
@@ -563,8 +611,9 @@ static hipError_t go_skinny_t(const GemvArgs &a, uint32_t waves, uint32_t ntiles
 }
 
 // One workgroup per CU at most, the tiles spread evenly over them, T of them
-// at a time (one per workgroup: 1, two: 2, more: 4, where two columns' operands
-// of two A tiles leave the registers for it, else 2).  C columns a wave, the
+// at a time (one per workgroup: 1, two: 2, more: 4, or 2 where two columns'
+// operands of two A tiles, or of one beside the sums' terms, leave no registers
+// for it: 20000x5120 at 8 rows 39 us with 4, which spill, 32 with 2).  C columns a wave, the
 // fewest that need no more than WMAX waves.
 template <class Q, bool HILO, int TOK, int WMAX, bool DB>
 static hipError_t go_skinny_w(const GemvArgs &a, hipStream_t s)
@@ -574,8 +623,9 @@ static hipError_t go_skinny_w(const GemvArgs &a, hipStream_t s)
     const uint32_t cus = device_cu_count(), per = (ntiles + cus - 1) / cus, grid = (ntiles + per - 1) / per;
     hipLaunchKernelGGL(skinny_encode_kernel<HILO>, dim3(B, TOK), dim3(256), 0, s, a.x, a.M, a.K, (uint8_t *)a.ws, (uint32_t)TOK);
     if (per == 1) return go_skinny_t<Q, HILO, TOK, 1, WMAX, DB>(a, waves, ntiles, grid, s);
-    if (per == 2 || (DB && TOK == 2)) return go_skinny_t<Q, HILO, TOK, 2, WMAX, DB>(a, waves, ntiles, grid, s);
-    return go_skinny_t<Q, HILO, TOK, DB && TOK == 2 ? 2 : 4, WMAX, DB>(a, waves, ntiles, grid, s);
+    constexpr bool few = DB && (TOK == 2 || Q::MINS);
+    if (per == 2 || few) return go_skinny_t<Q, HILO, TOK, 2, WMAX, DB>(a, waves, ntiles, grid, s);
+    return go_skinny_t<Q, HILO, TOK, few ? 2 : 4, WMAX, DB>(a, waves, ntiles, grid, s);
 }
 
 bool skinny_supported(const GemvArgs &a)
