@@ -637,13 +637,17 @@ bool skinny_supported(const GemvArgs &a)
     return a.w_bytes + RRR_READ_SLACK < SK_OOB;
 }
 
-// Waves a workgroup: up to 12 (168 registers a lane; 16 waves would leave 128,
-// and two columns' operands of one A tile spill), 8 where two columns' operands
-// of two A tiles are held.
+// Waves a workgroup: one a column to 12 columns, and to 16 with one A tile (16384 x
+// 4096 at 8 rows Q4_K 15.8 us against 20.6 with two columns a wave, Q6_K 20.1
+// against 21.8; 4096 x 4096 8.7 against 9.7); beyond, up to 12 (168 registers a
+// lane; 16 waves would leave 128, and two columns' operands of one A tile spill),
+// 8 where two columns' operands of two A tiles are held.
 template <class Q, bool HILO, int TOK>
 static hipError_t go_skinny(const GemvArgs &a, hipStream_t s)
 {
     if (a.K <= 12 * 256) return go_skinny_w<Q, HILO, TOK, 12, false>(a, s);
+    if constexpr (TOK == 1)
+        if (a.K <= 16 * 256) return go_skinny_w<Q, HILO, TOK, 16, false>(a, s);
     return go_skinny_w<Q, HILO, TOK, TOK == 1 ? 12 : 8, true>(a, s);
 }
 

@@ -66,3 +66,14 @@ def test_rows_of_any_size(ctx, qtype, K, N):
     ref = orc.gemv(qtype, raw, np.ascontiguousarray(X[fin]).reshape(-1), K, N, len(fin), 16, f64=True)
     for i, m in enumerate(fin):
         assert orc.normwise_err(Y[m], ref[i]) < F32_TOL, m
+
+
+@pytest.mark.parametrize("qtype,K,N", [(12, 4096, 4111), (13, 3328, 96), (14, 4096, 12300), (12, 4096, 16900)])
+@pytest.mark.parametrize("M", [3, 8])
+def test_rows_one_column_a_wave(ctx, qtype, K, N, M):
+    """13 to 16 columns with one A tile: one a wave, one to more than four tiles a workgroup."""
+    X = synth.normal_f32(26, M, M * K).reshape(M, K)
+    raw, Y = rows(ctx, qtype, K, N, X)
+    ref = orc.gemv(qtype, raw, X.reshape(-1), K, N, M, 16, f64=True)
+    for m in range(M):
+        assert orc.normwise_err(Y[m], ref[m]) < F32_TOL, m
