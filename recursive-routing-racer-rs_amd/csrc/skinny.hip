@@ -42,7 +42,8 @@
 // workgroup of the main kernel then loads its operands with 16-byte loads
 // instead of reading all of X in f32 and converting it again: at 8 rows QKV
 // 5120x3072 takes 9.5 us against 10.1 with the operands built in every wave,
-// gate+up 16384x3072 13.8 against 14.5.
+// gate+up 16384x3072 13.8 against 14.5.  Short rows are the other way round (see
+// go_skinny).
 //
 // Work split: a workgroup of W waves takes the 16-row tiles b, b + G, ... (G =
 // gridDim.x), T of them at a time; wave w owns the super-block columns w,
@@ -338,6 +339,28 @@ struct SkA {
     float pe[TOK][DPT];
 };
 
+// The same operands of one column and one A tile of 8 tokens built by the wave that
+// uses them, from its lane's values of the column (16 float4, two a sub-block):
+// the bits of skinny_encode_kernel.
+__device__ __forceinline__ void sk_build(SkA<1, 2> &x, const float4 (&xv)[16], uint32_t lane, uint32_t M)
+{
+    const uint32_t r16 = lane & 15, kg = lane >> 4;
+    const bool lo = r16 & 1, live = (r16 >> 1) < M;
+    float mx = 0.0f, gs[8];
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+        mx = fmaxf(mx, sk_max8(xv[2 * s], xv[2 * s + 1]));
+        gs[s] = lanes4_sum(sk_sum8(xv[2 * s], xv[2 * s + 1]));
+    }
+    const int e = sk_exponent(lanes4_max(mx));
+#pragma unroll
+    for (int s = 0; s < 8; s++) x.av[0][s] = sk_values(xv[2 * s], xv[2 * s + 1], e, lo, live);
+#pragma unroll
+    for (int i = 0; i < 4; i++) x.amin[0][i] = sk_half(kg == 0 ? gs[i] : gs[4 + i], e + 5, lo, live && kg < 2);
+#pragma unroll
+    for (int j = 0; j < 2; j++) x.pe[0][j] = ldexpf(1.0f, __shfl(e, 4 * kg + 2 * j, 64));
+}
+
 // Tile buffers a wave of a WMAX-wave workgroup gets out of the 160 KB of LDS.
 template <class Q, int WMAX>
 constexpr int sk_ring()
@@ -350,14 +373,16 @@ constexpr int sk_ring()
 // layout; T tiles at a time.  At most WMAX waves, NB = sk_ring tile buffers
 // per wave: units u + 1 .. u + NB - 1 stream in while unit u is multiplied
 // (unit = column, tile).  DB: more than one column a wave, the next column's A
-// operands requested one column ahead.
-template <class Q, bool HILO, int TOK, int T, int WMAX, bool DB>
+// operands requested one column ahead.  ENC: one column a wave, its A operands
+// built here instead of by the encoding pass.
+template <class Q, bool HILO, int TOK, int T, int WMAX, bool DB, bool ENC>
 __global__ __launch_bounds__(64 * WMAX) void skinny_kernel(GemvArgs a, uint32_t ntiles)
 {
     using G = SkGeom<Q>;
     constexpr int TPT = HILO ? 8 : 16, DPT = HILO ? 2 : 4, MP = TOK * TPT, NB = sk_ring<Q, WMAX>();
     constexpr int NA = DB ? TOK * (9 + (Q::MINS ? 1 : 0)) : 0;   // loads of one column's A operands
     constexpr int AHEAD = DB || NB - 1 < T ? NB - 1 : T;         // units issued before the first
+    static_assert(!ENC || (HILO && TOK == 1 && !DB), "operands built in the wave: one column, one A tile");
     static_assert(NB >= 2 && NB * G::BUF >= (uint32_t)T * MP * 64, "ring: two units, and the wave's row sums");
     extern __shared__ float smem[];
     const uint32_t K = a.K, M = a.M, N = a.N, B = K / 256, W = blockDim.x / 64;
@@ -550,14 +575,34 @@ __global__ __launch_bounds__(64 * WMAX) void skinny_kernel(GemvArgs a, uint32_t 
         }
     };
 
+    // the first units of the T tiles
+    auto start = [&] {
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) dma(u / T, tb0 + (u % T) * GR, u);
+    };
+    A x0, x1;
+    if constexpr (ENC) {
+        const float4 *xp = (const float4 *)(a.x + (uint64_t)min(r16 >> 1, M - 1) * K + wave * 256 + 8 * kg);
+        float4 xv[16];
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            xv[2 * s] = xp[8 * s];
+            xv[2 * s + 1] = xp[8 * s + 1];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        start();
+        sk_build(x0, xv, lane, M);
+    }
     for (; tb0 < ntiles; tb0 += T * GR) {
         // the first columns' A operands, then the first units: loads return in
         // order, so unit 0 waits for the A operands and its own weights only
-        A x0, x1;
-        load_a(x0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 0; u < AHEAD; u++) dma(u / T, tb0 + (u % T) * GR, u);
+        if constexpr (!ENC) {
+            load_a(x0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            start();
+        } else if (tb0 != tile0) {
+            start();
+        }
 #pragma unroll
         for (int ti = 0; ti < T; ti++)
 #pragma unroll
@@ -602,11 +647,11 @@ __global__ __launch_bounds__(64 * WMAX) void skinny_kernel(GemvArgs a, uint32_t 
     }
 }
 
-template <class Q, bool HILO, int TOK, int T, int WMAX, bool DB>
+template <class Q, bool HILO, int TOK, int T, int WMAX, bool DB, bool ENC>
 static hipError_t go_skinny_t(const GemvArgs &a, uint32_t waves, uint32_t ntiles, uint32_t grid, hipStream_t s)
 {
     const size_t lds = (size_t)waves * sk_ring<Q, WMAX>() * SkGeom<Q>::BUF;
-    hipLaunchKernelGGL((skinny_kernel<Q, HILO, TOK, T, WMAX, DB>), dim3(grid), dim3(64 * waves), lds, s, a, ntiles);
+    hipLaunchKernelGGL((skinny_kernel<Q, HILO, TOK, T, WMAX, DB, ENC>), dim3(grid), dim3(64 * waves), lds, s, a, ntiles);
     return hipGetLastError();
 }
 
@@ -615,17 +660,18 @@ static hipError_t go_skinny_t(const GemvArgs &a, uint32_t waves, uint32_t ntiles
 // operands of two A tiles, or of one beside the sums' terms, leave no registers
 // for it: 20000x5120 at 8 rows 39 us with 4, which spill, 32 with 2).  C columns a wave, the
 // fewest that need no more than WMAX waves.
-template <class Q, bool HILO, int TOK, int WMAX, bool DB>
+template <class Q, bool HILO, int TOK, int WMAX, bool DB, bool ENC = false>
 static hipError_t go_skinny_w(const GemvArgs &a, hipStream_t s)
 {
     const uint32_t B = a.K / 256, ntiles = (a.N + 15) / 16;
     const uint32_t C = (B + WMAX - 1) / WMAX, waves = (B + C - 1) / C;
     const uint32_t cus = device_cu_count(), per = (ntiles + cus - 1) / cus, grid = (ntiles + per - 1) / per;
-    hipLaunchKernelGGL(skinny_encode_kernel<HILO>, dim3(B, TOK), dim3(256), 0, s, a.x, a.M, a.K, (uint8_t *)a.ws, (uint32_t)TOK);
-    if (per == 1) return go_skinny_t<Q, HILO, TOK, 1, WMAX, DB>(a, waves, ntiles, grid, s);
+    if constexpr (!ENC)
+        hipLaunchKernelGGL(skinny_encode_kernel<HILO>, dim3(B, TOK), dim3(256), 0, s, a.x, a.M, a.K, (uint8_t *)a.ws, (uint32_t)TOK);
+    if (per == 1) return go_skinny_t<Q, HILO, TOK, 1, WMAX, DB, ENC>(a, waves, ntiles, grid, s);
     constexpr bool few = DB && (TOK == 2 || Q::MINS);
-    if (per == 2 || few) return go_skinny_t<Q, HILO, TOK, 2, WMAX, DB>(a, waves, ntiles, grid, s);
-    return go_skinny_t<Q, HILO, TOK, few ? 2 : 4, WMAX, DB>(a, waves, ntiles, grid, s);
+    if (per == 2 || few) return go_skinny_t<Q, HILO, TOK, 2, WMAX, DB, ENC>(a, waves, ntiles, grid, s);
+    return go_skinny_t<Q, HILO, TOK, few ? 2 : 4, WMAX, DB, ENC>(a, waves, ntiles, grid, s);
 }
 
 bool skinny_supported(const GemvArgs &a)
@@ -642,12 +688,18 @@ bool skinny_supported(const GemvArgs &a)
 // against 21.8; 4096 x 4096 8.7 against 9.7); beyond, up to 12 (168 registers a
 // lane; 16 waves would leave 128, and two columns' operands of one A tile spill),
 // 8 where two columns' operands of two A tiles are held.
+// To 8 columns and 8 rows the waves build their own operands: the pass costs a
+// launch, the building in every wave a chain of ~600 instructions that waits on
+// x (5 rows, 1024 to 5632 weight rows, K = 1024 4.2 to 4.9 us against 5.5 to 6.4 with the
+// pass, 2048 5.8 to 7.0 against 6.3 to 7.5, 2560 7.3 to 8.9 against 6.9 to 8.5).
 template <class Q, bool HILO, int TOK>
 static hipError_t go_skinny(const GemvArgs &a, hipStream_t s)
 {
+    if constexpr (TOK == 1) {
+        if (a.K <= 8 * 256) return go_skinny_w<Q, HILO, TOK, 8, false, true>(a, s);
+        if (a.K > 12 * 256 && a.K <= 16 * 256) return go_skinny_w<Q, HILO, TOK, 16, false>(a, s);
+    }
     if (a.K <= 12 * 256) return go_skinny_w<Q, HILO, TOK, 12, false>(a, s);
-    if constexpr (TOK == 1)
-        if (a.K <= 16 * 256) return go_skinny_w<Q, HILO, TOK, 16, false>(a, s);
     return go_skinny_w<Q, HILO, TOK, TOK == 1 ? 12 : 8, true>(a, s);
 }
 

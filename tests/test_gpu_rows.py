@@ -77,3 +77,23 @@ def test_rows_one_column_a_wave(ctx, qtype, K, N, M):
     ref = orc.gemv(qtype, raw, X.reshape(-1), K, N, M, 16, f64=True)
     for m in range(M):
         assert orc.normwise_err(Y[m], ref[m]) < F32_TOL, m
+
+
+@pytest.mark.parametrize("qtype,K,N", [(14, 256, 16), (12, 256, 8200), (13, 1024, 4111), (14, 1280, 12300),
+                                       (12, 2048, 20000), (13, 2048, 100)])
+def test_operands_built_in_the_wave(ctx, qtype, K, N):
+    """To 8 columns and 8 rows a wave builds its operands itself: bit for bit those of the encoding pass, which calls
+    of more rows take (two A tiles; the same products and sums for each row)."""
+    X = synth.normal_f32(30, 1, 12 * K).reshape(12, K)
+    X[1] *= np.float32(1e30)
+    X[2] *= np.float32(1e-36)
+    X[3] = 0.0
+    X[4, ::7] *= np.float32(100.0)
+    Y12 = rows(ctx, qtype, K, N, X)[1]
+    for M in (5, 7, 8):
+        raw, Y = rows(ctx, qtype, K, N, X[:M].copy())
+        assert np.array_equal(Y.view(np.uint32), Y12[:M].view(np.uint32)), M
+    ref = orc.gemv(qtype, raw, X[:8].reshape(-1), K, N, 8, 16, f64=True)
+    for m in (0, 1, 4, 5, 6, 7):
+        assert orc.normwise_err(Y[m], ref[m]) < F32_TOL, m
+    assert np.all(Y[3] == 0.0)
