@@ -599,17 +599,36 @@ static bool batched_gemm_route(const GemvArgs &a)
            gemm_rows_supported(a.type, a.K, a.N, a.M, a.ws_bytes);
 }
 
+// Long rows of few weights, where the VALU kernel's workgroups (8 weight rows and 2
+// token rows, 4 from 4 token rows on) cover the CUs at most once and its time is
+// one workgroup's walk along K; the skinny kernel has an eighth of the workgroups
+// for the same walk.  2 and 3 rows, us, VALU (skinny): 1024x4096 Q6_K 6.9 (9.5),
+// 1024x6144 Q4_K 8.2 (11.0), 1024x8192 Q5_K 11.8 (13.6), 512x10240 Q4_K 12.1
+// (14.0), 2048x16384 Q4_K 18.8 (20.2), but 28672 columns 28.7 (27.1), and 33
+// columns 12.5 (12.4): a last chunk of few columns costs as much as half a chunk.  9
+// to 16 rows: 512x4096 Q4_K 9.9 (10.8), Q5_K 10.7 (11.4), 512x6144 13.4 (13.3),
+// Q6_K 13.2 (12.1).
+static bool valu_rows(const GemvArgs &a)
+{
+    const uint32_t mt = a.M >= 4 ? 4 : 2;
+    if (a.type == T_F32 || (uint64_t)((a.M + mt - 1) / mt) * ((a.N + 7) / 8) > device_cu_count()) return false;
+    if (a.M <= 3) return a.K > 3072 && a.K <= 16384 && (a.K % 4096 == 0 || a.K % 4096 >= 1024);
+    return a.M > 8 && a.M <= 16 && a.type != T_Q6_K && a.K > 3072 && a.K <= 5120;
+}
+
 // M > 1 rows of plain activations.  2 to 4 rows: the int8 GEMV's multi-token
 // form where it applies (K <= 3072, 2 rows to 8192).  To 16 rows: the skinny
-// kernel with hi/lo activations, f32 accuracy.  17 to 32 rows: the skinny
+// kernel with hi/lo activations, f32 accuracy (few weights and long rows: the VALU
+// kernel).  17 to 32 rows: the skinny
 // kernel with f16 activations where such rows may be f16 (Q4_K / Q5_K with
 // K <= 3072, and what the GEMM takes); the GEMM above 32.  Where they may not
 // (N not a multiple of 64, unaligned rows), 16 rows at a time with hi/lo
-// activations.  Returns hipErrorNotSupported for what only the VALU kernels
-// take (F32 weights, tensors of 2 GB).
+// activations.  Returns hipErrorNotSupported for what the VALU kernels take
+// (those, F32 weights, tensors of 2 GB).
 static hipError_t launch_rows(const GemvArgs &a, hipStream_t s)
 {
     if (gemv_mq_tokens_supported(a)) return launch_gemv_mq_tokens(a, s);
+    if (valu_rows(a)) return hipErrorNotSupported;
     const bool gemm = batched_gemm_route(a);
     if (skinny_supported(a) && (a.M <= 16 || gemm || (a.type != T_Q6_K && a.K <= 3072))) return launch_skinny(a, s);
     if (gemm) return launch_gemm_f32_rows(a.x, a.W, a.type, a.y, a.K, a.N, a.M, a.ws, a.ws_bytes, a.wx, s);

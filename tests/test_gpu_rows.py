@@ -97,3 +97,16 @@ def test_operands_built_in_the_wave(ctx, qtype, K, N):
     for m in (0, 1, 4, 5, 6, 7):
         assert orc.normwise_err(Y[m], ref[m]) < F32_TOL, m
     assert np.all(Y[3] == 0.0)
+
+
+@pytest.mark.parametrize("qtype,K,N,M", [
+    (14, 4096, 1024, 3), (12, 6144, 1000, 3), (13, 8192, 2048, 2), (14, 16384, 16, 2),      # VALU kernel
+    (12, 4096, 512, 16), (13, 5120, 680, 12), (12, 3328, 500, 9),
+    (14, 4096, 1032, 3), (12, 16640, 64, 3), (12, 12544, 64, 2), (14, 4096, 512, 16), (12, 5376, 512, 16)])   # past it
+def test_long_rows_of_few_weights(ctx, qtype, K, N, M):
+    """Both sides of the rule that leaves few weights and long rows to the VALU kernel."""
+    X = synth.normal_f32(32, M, M * K).reshape(M, K)
+    raw, Y = rows(ctx, qtype, K, N, X)
+    ref = orc.gemv(qtype, raw, X.reshape(-1), K, N, M, 16, f64=True)
+    for m in range(M):
+        assert orc.normwise_err(Y[m], ref[m]) < F32_TOL, m
