@@ -80,7 +80,13 @@ typedef struct rrr_graph rrr_graph;
  * context's stream.  device == RRR_DEVICE_NONE creates a validation-only
  * context: buffers are placeholders with a size and no memory, every call
  * validates its arguments as usual and then returns RRR_ERR_NO_DEVICE instead
- * of touching a GPU. */
+ * of touching a GPU.
+ * A context holds about 180 MiB of device memory from here to rrr_destroy: 48
+ * MiB of GEMM workspace (partials, converted rows), 128 MiB for weights expanded
+ * to f16 by the GEMMs of long prompts, a few of attention scratch; and 256 KiB
+ * of pinned host memory for rrr_matmul_kquant.  Where there is no room for the
+ * 128 MiB or the pinned memory the context does without: the calls that would
+ * use them take their other forms. */
 #define RRR_DEVICE_NONE (-1)
 int rrr_init(int device, rrr_ctx **out);
 /* Replaces Drop for ComputeEngine (engine.rs:557-579): waits for the device,

@@ -58,6 +58,12 @@ int rrr_probe_mfma(rrr_ctx *ctx, uint32_t kind, uint32_t waves_per_cu, uint32_t 
 /* CUs of the context's device (the probes' grid unit); 0 without a device. */
 uint32_t rrr_probe_cus(rrr_ctx *ctx);
 
+/* Gives back what a context allocates only to make calls faster (the 128 MiB of
+ * expanded weights of the long-prompt GEMM, the pinned staging of
+ * rrr_matmul_kquant): the context is then as rrr_init leaves it where there
+ * is no room for them.  Graphs recorded before must not be launched after. */
+int rrr_probe_drop_optional(rrr_ctx *ctx);
+
 #ifdef __cplusplus
 }
 #endif

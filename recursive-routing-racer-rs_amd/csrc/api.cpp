@@ -86,8 +86,9 @@ struct rrr_ctx {
     void *att_scratch;  // attention: per-KV-head counters (zero between calls) and split partials
     void *gemm_ws;      // GEMM_WS_BYTES: prefill GEMM partials of split K; the skinny GEMV's encoded
                         // activations; the split-K logits' partials (stream order keeps the users apart)
-    void *gemm_wx;      // GEMM_WX_BYTES: weights expanded to f16 for the long-prompt GEMM
-    float *pin;         // pinned host staging of rrr_matmul_kquant: PIN_FLOATS in, PIN_FLOATS out
+    void *gemm_wx;      // GEMM_WX_BYTES: weights expanded to f16 for the long-prompt GEMM; null where the
+                        // device has no room for it: that GEMM is then never taken
+    float *pin;         // pinned host staging of rrr_matmul_kquant: PIN_FLOATS in, PIN_FLOATS out; null: none
     void *logits_cnt;   // split-K logits: per-slab counters (zero between calls)
     std::unordered_set<rrr_buf *> bufs;
     std::unordered_set<rrr_graph *> graphs;
@@ -213,8 +214,15 @@ int rrr_init(int device, rrr_ctx **out)
         if (e == hipSuccess) e = hipMalloc(&ctx->att_scratch, attention_scratch_bytes());
         if (e == hipSuccess) e = hipMemset(ctx->att_scratch, 0, attention_scratch_bytes());
         if (e == hipSuccess) e = hipMalloc(&ctx->gemm_ws, GEMM_WS_BYTES);
-        if (e == hipSuccess) e = hipMalloc(&ctx->gemm_wx, GEMM_WX_BYTES);
-        if (e == hipSuccess) e = hipHostMalloc((void **)&ctx->pin, 2ull * PIN_FLOATS * 4, hipHostMallocMapped);
+        // what only makes calls faster, a context does without
+        if (e == hipSuccess && hipMalloc(&ctx->gemm_wx, GEMM_WX_BYTES) != hipSuccess) {
+            ctx->gemm_wx = nullptr;
+            (void)hipGetLastError();
+        }
+        if (e == hipSuccess && hipHostMalloc((void **)&ctx->pin, 2ull * PIN_FLOATS * 4, hipHostMallocMapped) != hipSuccess) {
+            ctx->pin = nullptr;
+            (void)hipGetLastError();
+        }
         if (e == hipSuccess) e = hipMalloc(&ctx->logits_cnt, logits_counter_bytes());
         if (e == hipSuccess) e = hipMemset(ctx->logits_cnt, 0, logits_counter_bytes());
         if (e == hipSuccess) e = hipDeviceSynchronize();
@@ -264,8 +272,8 @@ int rrr_destroy(rrr_ctx *ctx)
         (void)hipFree(ctx->scratch);
         (void)hipFree(ctx->att_scratch);
         (void)hipFree(ctx->gemm_ws);
-        (void)hipFree(ctx->gemm_wx);
-        (void)hipHostFree(ctx->pin);
+        if (ctx->gemm_wx) (void)hipFree(ctx->gemm_wx);
+        if (ctx->pin) (void)hipHostFree(ctx->pin);
         (void)hipFree(ctx->logits_cnt);
         (void)hipEventDestroy(ctx->ev0);
         (void)hipEventDestroy(ctx->ev1);
@@ -1461,6 +1469,21 @@ uint32_t rrr_probe_cus(rrr_ctx *ctx)
     return device_cu_count();
 }
 
+int rrr_probe_drop_optional(rrr_ctx *ctx)
+{
+    TRY(check_ctx(ctx));
+    const char *what = "rrr_probe_drop_optional";
+    if (ctx->capturing) return fail(RRR_ERR_STATE, "%s: not allowed during capture", what);
+    TRY(device_ready(ctx));
+    hipError_t e = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess && ctx->gemm_wx) e = hipFree(ctx->gemm_wx);
+    if (e == hipSuccess && ctx->pin) e = hipHostFree(ctx->pin);
+    if (e != hipSuccess) return fail(RRR_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
+    ctx->gemm_wx = nullptr;
+    ctx->pin = nullptr;
+    return ok();
+}
+
 // ---- one-call helper ------------------------------------------------------------
 
 int rrr_matmul_kquant(rrr_ctx *ctx, rrr_buf *buf_a, const rrr_buf *weight_buf, rrr_buf *buf_c, uint32_t type,
@@ -1482,7 +1505,7 @@ int rrr_matmul_kquant(rrr_ctx *ctx, rrr_buf *buf_a, const rrr_buf *weight_buf, r
     // that copy, GEMV and copy run back to back with one wait at the end; a
     // pageable hipMemcpyAsync and a wait each way took most of the call
     // (Q6_K 3072x8192: 53 -> 25 us, of which the GEMV is 8).
-    const bool staged = K <= PIN_FLOATS && N <= PIN_FLOATS && !ctx->nodevice;
+    const bool staged = ctx->pin && K <= PIN_FLOATS && N <= PIN_FLOATS;
     if (staged) {
         TRY(device_ready(ctx));
         memcpy(ctx->pin, a, (size_t)K * 4);

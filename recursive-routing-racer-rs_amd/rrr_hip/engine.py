@@ -317,6 +317,9 @@ class Context:
     def probe_cus(self):
         return int(self.lib.rrr_probe_cus(self._h))
 
+    def probe_drop_optional(self):
+        _check(self.lib.rrr_probe_drop_optional(self._h))
+
     def sync(self):
         _check(self.lib.rrr_sync(self._h))
 
