@@ -58,6 +58,11 @@ int rrr_probe_mfma(rrr_ctx *ctx, uint32_t kind, uint32_t waves_per_cu, uint32_t 
 /* CUs of the context's device (the probes' grid unit); 0 without a device. */
 uint32_t rrr_probe_cus(rrr_ctx *ctx);
 
+/* The form rrr_gemm_f16 takes for M rows: *wide_tile = the tile columns of the GEMM
+ * on expanded weights, *splits = 1, or *wide_tile = 0 and the splits of K of the
+ * GEMM that dequantizes as it goes.  Needs no device. */
+int rrr_probe_gemm_route(rrr_ctx *ctx, uint32_t K, uint32_t N, uint32_t M, uint32_t *wide_tile, uint32_t *splits);
+
 /* Gives back what a context allocates only to make calls faster (the 128 MiB of
  * expanded weights of the long-prompt GEMM, the pinned staging of
  * rrr_matmul_kquant): the context is then as rrr_init leaves it where there

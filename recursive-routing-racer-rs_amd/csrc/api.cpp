@@ -1469,6 +1469,20 @@ uint32_t rrr_probe_cus(rrr_ctx *ctx)
     return device_cu_count();
 }
 
+int rrr_probe_gemm_route(rrr_ctx *ctx, uint32_t K, uint32_t N, uint32_t M, uint32_t *wide_tile, uint32_t *splits)
+{
+    TRY(check_ctx(ctx));
+    const char *what = "rrr_probe_gemm_route";
+    if (!wide_tile || !splits) return fail(RRR_ERR_NULL, "%s: null output pointer", what);
+    TRY(check_shape(T_Q4_K, K, N));
+    if (!M || !gemm_supported(T_Q4_K, K, N, M, (uint64_t)M * K * 2))
+        return fail(RRR_ERR_UNSUPPORTED, "%s: needs M %% 128 == 0 and N %% 64 == 0 (M=%u N=%u)", what, M, N);
+    const GemmRoute r = gemm_route(K, N, M, M, GEMM_WS_BYTES, ctx->nodevice || ctx->gemm_wx);
+    *wide_tile = r.wide_tile;
+    *splits = r.splits;
+    return ok();
+}
+
 int rrr_probe_drop_optional(rrr_ctx *ctx)
 {
     TRY(check_ctx(ctx));

@@ -709,6 +709,16 @@ bool gemm_supported(uint32_t type, uint32_t K, uint32_t N, uint32_t M, uint64_t 
            (uint64_t)N * (K / 256) * 210 + RRR_READ_SLACK < GM_OOB && x_bytes + RRR_READ_SLACK < GM_OOB;
 }
 
+GemmRoute gemm_route(uint32_t K, uint32_t N, uint32_t M, uint32_t mrows, size_t split_bytes, bool wide)
+{
+    const GemmPlan p = gemm_plan(K, N, M, split_bytes != 0, split_bytes);
+    // the weights expanded to f16 first where that is faster: long prompts,
+    // and row counts that leave the 256 x 128 tiles' rounds part empty
+    if (wide && gemm_wide_cost(K, N, mrows, GEMM_WX_BYTES) < 0.97f * p.us)
+        return {gemm_wide_tile(K, N, mrows, GEMM_WX_BYTES), 1u};
+    return {0u, p.S};
+}
+
 template <bool ACC>
 static hipError_t go_gemm_q(const uint16_t *X, const float *rscale, const uint8_t *W, uint32_t type, float *Y,
                             uint32_t K, uint32_t N, uint32_t M, uint32_t mrows, float *ws, size_t ws_bytes, void *wx,
@@ -717,9 +727,7 @@ static hipError_t go_gemm_q(const uint16_t *X, const float *rscale, const uint8_
     if (!gemm_supported(type, K, N, M, (uint64_t)M * K * 2) || mrows == 0 || mrows > M) return hipErrorNotSupported;
     // the fused reductions and what follows take every one of the M rows
     if ((nrm || rp) && mrows != M) return hipErrorInvalidValue;
-    // the weights expanded to f16 first where that is faster: long prompts,
-    // and row counts that leave the 256 x 128 tiles' rounds part empty
-    if (wx && gemm_wide_cost(K, N, mrows, GEMM_WX_BYTES) < 0.97f * gemm_plan(K, N, M, ws != nullptr, ws_bytes).us) {
+    if (gemm_route(K, N, M, mrows, ws ? ws_bytes : 0, wx != nullptr).wide_tile) {
         const hipError_t e = launch_gemm_wide(X, rscale, W, type, Y, K, N, M, mrows, ACC, wx, GEMM_WX_BYTES, s);
         return e == hipSuccess ? gemm_then(Y, N, M, nrm, rp, s) : e;
     }

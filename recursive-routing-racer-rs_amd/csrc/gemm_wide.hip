@@ -1,5 +1,6 @@
 // gemm_wide.hip -- the prefill GEMM for long prompts: Y[M][N] = X[M][K] . W[N][K]^T
-// (or Y +=) with X in f16 and W first expanded to f16, once per call.
+// (or Y +=) with X in f16 and W first expanded to f16, once per launch of the
+// GEMM (once per chunk of rows where a call's rows go through the workspace).
 //
 // gemm_dq_kernel (gemm.hip) dequantizes a weight tile again for every 256 rows
 // of X, with half of its waves, and its 256 x 128 tiles leave the last round of
@@ -330,6 +331,12 @@ static uint32_t gw_best(uint32_t K, uint32_t N, uint32_t M)
     for (uint32_t bn : {192u, 160u, 128u, 96u, 64u})
         if (gw_cost(K, N, M, bn) < gw_cost(K, N, M, best)) best = bn;
     return best;
+}
+
+uint32_t gemm_wide_tile(uint32_t K, uint32_t N, uint32_t M, size_t wx_bytes)
+{
+    const uint32_t c = gw_cols(K, N, wx_bytes);
+    return c ? gw_best(K, c < N ? c : N, M) : 0;
 }
 
 float gemm_wide_cost(uint32_t K, uint32_t N, uint32_t M, size_t wx_bytes)

@@ -173,11 +173,20 @@ inline float gemm_rounds(uint32_t tiles, float base, float load, float fixed)
 }
 // The same product with W expanded to f16 first (gemm_wide.hip), whole K: the
 // bits of launch_gemm_f16 without split K.  mrows <= M: the rows stored.
-// gemm_wide_cost: its time in us, for the choice between the two.
+// gemm_wide_cost: its time in us, for the choice between the two; gemm_wide_tile:
+// the columns of its tiles (0: not taken), of its first column part.
+uint32_t gemm_wide_tile(uint32_t K, uint32_t N, uint32_t M, size_t wx_bytes);
 float gemm_wide_cost(uint32_t K, uint32_t N, uint32_t M, size_t wx_bytes);
 hipError_t launch_gemm_wide(const uint16_t *X, const float *rscale, const uint8_t *W, uint32_t type, float *Y,
                             uint32_t K, uint32_t N, uint32_t M, uint32_t mrows, bool acc, void *wx, size_t wx_bytes,
                             hipStream_t s);
+// The form a GEMM of `mrows` of M rows takes: the wide one's tile columns, or 0 and
+// the splits of K.  split_bytes: workspace for split partials (0: no split);
+// wide: there is a workspace for expanded weights.
+struct GemmRoute {
+    uint32_t wide_tile, splits;
+};
+GemmRoute gemm_route(uint32_t K, uint32_t N, uint32_t M, uint32_t mrows, size_t split_bytes, bool wide);
 // the same GEMM, then the RMSNorm (gamma, eps) of Y's rows in f16 into out16:
 // with K split, inside the split reduction (splitk_reduce_rmsnorm_kernel),
 // else the rmsnorm launch after the GEMM; N % 4 == 0, N <= 8192

@@ -102,6 +102,7 @@ SIGNATURES = {
                                     c_buf_p, ctypes.POINTER(u32), ctypes.POINTER(u32)]),
     "rrr_probe_mfma": (i32, [c_ctx_p, u32, u32, u32, c_buf_p]),
     "rrr_probe_cus": (u32, [c_ctx_p]),
+    "rrr_probe_gemm_route": (i32, [c_ctx_p, u32, u32, u32, ctypes.POINTER(u32), ctypes.POINTER(u32)]),
     "rrr_probe_drop_optional": (i32, [c_ctx_p]),
     "rrr_rope_kv_store_rows": (i32, [c_ctx_p, c_buf_p, u32, c_buf_p, u32, c_buf_p, c_buf_p, u32, u32, u32, u32, u32,
                                      u32, u32, f32, f32]),

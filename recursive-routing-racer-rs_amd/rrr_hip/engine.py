@@ -317,6 +317,12 @@ class Context:
     def probe_cus(self):
         return int(self.lib.rrr_probe_cus(self._h))
 
+    def probe_gemm_route(self, K, N, M):
+        """(tile columns of the GEMM on expanded weights or 0, splits of K) of rrr_gemm_f16."""
+        t, s = ctypes.c_uint32(), ctypes.c_uint32()
+        _check(self.lib.rrr_probe_gemm_route(self._h, K, N, M, ctypes.byref(t), ctypes.byref(s)))
+        return t.value, s.value
+
     def probe_drop_optional(self):
         _check(self.lib.rrr_probe_drop_optional(self._h))
 
