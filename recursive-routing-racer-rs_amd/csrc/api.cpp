@@ -466,7 +466,7 @@ int rrr_dequant(rrr_ctx *ctx, uint32_t type, const rrr_buf *W, rrr_buf *out, uin
     TRY(need(W, n / 256 * block_bytes(type), "rrr_dequant W"));
     TRY(need_f32(out, n, "rrr_dequant out"));
     TRY(device_ready(ctx));
-    return finish(ctx, launch_dequant(type, (const uint8_t *)W->ptr, W->bytes, (float *)out->ptr, n, ctx->stream),
+    return finish(ctx, launch_dequant(type, (const uint8_t *)W->ptr, (float *)out->ptr, n, ctx->stream),
                   "rrr_dequant");
 }
 

@@ -85,7 +85,8 @@ hipError_t launch_rope_kv_store(float *qkv, const RopeArgs &r, uint16_t *kc, uin
 // followed by rope_kv_store_kernel.  Rows m >= rows (the GEMM's padding rows)
 // get the plain sums.  A thread takes two quads of elements (two pairs each) a
 // pass, and the launcher as many threads as make one pass of the row up to 8,192
-// elements: bound by latency at a few rows (the partials' round trip and the
+// elements (4,096 with 7 or 8 splits, whose partials leave registers for 512
+// threads): bound by latency at a few rows (the partials' round trip and the
 // coefficients' powf and sincosf, which the requests now overlap), by HBM at
 // many.  128 rows of 5,120 at three splits 7.0 -> 4.9 us against 256 threads and
 // five dependent passes, 512 rows 11.2 in both.  The launcher requires q_dim,

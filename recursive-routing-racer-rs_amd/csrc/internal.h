@@ -78,8 +78,7 @@ bool skinny_supported(const GemvArgs &a);
 hipError_t launch_skinny(const GemvArgs &a, hipStream_t s);
 // CUs of the current device (cached per device)
 uint32_t device_cu_count();
-hipError_t launch_dequant(uint32_t type, const uint8_t *W, uint64_t w_bytes, float *out,
-                          uint64_t n_elements, hipStream_t s);
+hipError_t launch_dequant(uint32_t type, const uint8_t *W, float *out, uint64_t n, hipStream_t s);
 hipError_t launch_rmsnorm(const float *x, const float *g, float *y, uint32_t rows, uint32_t d,
                           float eps, hipStream_t s);
 hipError_t launch_silu_gate(const float *gu, float *mid, uint32_t rows, uint32_t F, hipStream_t s);

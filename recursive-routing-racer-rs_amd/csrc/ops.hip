@@ -92,8 +92,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t *__restrict_
         if (b0 + i < n_blocks) __builtin_nontemporal_store(r[i].values(lane), (f32x4 *)(out + (b0 + i) * 256) + lane);
 }
 
-hipError_t launch_dequant(uint32_t type, const uint8_t *W, uint64_t w_bytes, float *out, uint64_t n,
-                          hipStream_t s)
+hipError_t launch_dequant(uint32_t type, const uint8_t *W, float *out, uint64_t n, hipStream_t s)
 {
     const uint64_t nb = n / 256;
     const dim3 grid((unsigned)((nb + 4 * DQ_BLOCKS - 1) / (4 * DQ_BLOCKS)));
