@@ -25,7 +25,8 @@ CASES = [(64, 1536, 1088, 2048), (64, 256, 8192, 1408),
          (128, 512, 4160, 1536), (128, 512, 5696, 1152), (128, 3072, 5120, 1152),
          (160, 256, 5184, 1664), (160, 3072, 5120, 1920),
          (192, 256, 5184, 2048), (192, 256, 5696, 1920), (192, 3072, 16384, 1152),
-         (256, 256, 9024, 1408), (256, 256, 16448, 768), (256, 3072, 8192, 1536)]
+         (256, 256, 9024, 1408), (256, 256, 16448, 768), (256, 3072, 8192, 1536),
+         (96, 10240, 8192, 1152)]     # 160 MiB of f16 weights: two column parts
 
 
 @pytest.mark.parametrize("tile,K,N,M", CASES)
