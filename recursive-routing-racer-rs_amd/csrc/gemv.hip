@@ -601,8 +601,8 @@ static bool batched_gemm_route(const GemvArgs &a)
 
 // Long rows of few weights, where the VALU kernel's workgroups (8 weight rows and 2
 // token rows, 4 from 4 token rows on) cover the CUs at most once and its time is
-// one workgroup's walk along K; the skinny kernel has an eighth of the workgroups
-// for the same walk.  2 and 3 rows, us, VALU (skinny): 1024x4096 Q6_K 6.9 (9.5),
+// one workgroup's walk along K; the skinny kernel has half (2 rows) to an eighth
+// (16 rows) of the workgroups for the same walk.  2 and 3 rows, us, VALU (skinny): 1024x4096 Q6_K 6.9 (9.5),
 // 1024x6144 Q4_K 8.2 (11.0), 1024x8192 Q5_K 11.8 (13.6), 512x10240 Q4_K 12.1
 // (14.0), 2048x16384 Q4_K 18.8 (20.2), but 28672 columns 28.7 (27.1), and 33
 // columns 12.5 (12.4): a last chunk of few columns costs as much as half a chunk.  9
