@@ -65,7 +65,8 @@
 //
 // Bound: HBM at every M in principle (20.6 MB of Q6_K in 2.9 us); in fact a CU's
 // intake (at K = 8192 and 8 rows 262 KB of A operands next to its 80 KB of
-// weights) and the decode (~330 VALU instructions a unit, three waves a SIMD).
+// weights) and the decode (counted at 8 rows: 200 VALU instructions a unit of 16
+// columns x 256 for Q4_K, 240 for Q5_K; three waves a SIMD).
 // Measured per call, graphs over 300 MB of weight copies, in us, against the
 // VALU kernel (four rows a pass over the weights) and, at 27 rows, the row
 // conversion + prefill GEMM + split reduction that took these shapes before:
